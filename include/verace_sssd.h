@@ -83,7 +83,11 @@ int vmi_sssd_scan_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D,
  *   out      may be NULL if only the final state is wanted.
  * Supported: io_dtype in {F32, BF16, F16}; delta_dtype in {F32, BF16, F16};
  * 1 <= D <= 256.  T = 0 copies psi_in (or identity) to psi_out.
- * Arithmetic: F32 I/O, D != 128 and T < 32 run in fp32 token by token.  BF16 / F16 I/O with
+ * Arithmetic: F32 I/O, D != 128 and T < 32 run in fp32: in chunks of 16 tokens on the fp32
+ * matrix cores for 5 <= T and D <= 128, given the workspace of vmi_sssd_scan_workspace_bytes
+ * (optional for these calls: without it, or with less, they run token by token, as T < 5,
+ * D > 128 and any sequence with a rotation m > 0.25 or a non-finite token always do).
+ * BF16 / F16 I/O with
  * D = 128 and T >= 32 run the chunk-parallel scan, whose matrix-core operands (the state, W
  * and Z, once per 16-token chunk) are f16 with fp32 accumulation.  That holds the 2e-2
  * relative / 1e-4 norm-drift bars while every token's rotation

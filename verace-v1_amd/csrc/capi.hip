@@ -93,7 +93,7 @@ int vmi_sssd_scan_fwd(const void* q, const void* k, const void* v, const void* d
   const size_t state_bytes = static_cast<size_t>(B * H) * D * D * sizeof(float);
   if (psi_in != nullptr && ranges_overlap(psi_in, state_bytes, psi_out, state_bytes))
     return VMI_ERR_ALIAS;
-  const size_t need = vmi::scan_workspace_bytes(B, T, H, D, io_dtype);
+  const size_t need = vmi::scan_workspace_required(B, T, H, D, io_dtype);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) return VMI_ERR_WORKSPACE;
   if (B == 0 || H == 0) return VMI_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -64,16 +64,17 @@ extern "C" int vmi_sssd_scan_fwd_noalloc(const void* q, const void* k, const voi
     const char* b = reinterpret_cast<const char*>(psi_out);
     if (a < b + state_bytes && b < a + state_bytes) return VMI_ERR_ALIAS;
   }
-  const size_t need = vmi::scan_workspace_bytes(B, T, H, D, io_dtype);
-  if (need > kScratchBytes) return VMI_ERR_WORKSPACE;  // beyond the fixed array: use vmi_sssd_scan_fwd
+  if (vmi::scan_workspace_required(B, T, H, D, io_dtype) > kScratchBytes) return VMI_ERR_WORKSPACE;  // beyond the fixed array: use vmi_sssd_scan_fwd
   if (B == 0 || H == 0) return VMI_OK;
   void* ws = nullptr;
-  if (need > 0) {
+  const size_t want = vmi::scan_workspace_bytes(B, T, H, D, io_dtype);
+  if (want > 0 && want <= kScratchBytes) {  // a larger optional workspace: run without
     const hipError_t e = scratch_address(&ws);
     if (e != hipSuccess) return vmi::hip_status(e);
   }
   return vmi::hip_status(vmi::dispatch_scan(q, k, v, delta, io_dtype, delta_dtype, psi_in, out,
                                             psi_out, static_cast<int>(B), static_cast<int>(T),
-                                            static_cast<int>(H), static_cast<int>(D), ws, need,
+                                            static_cast<int>(H), static_cast<int>(D), ws,
+                                            ws != nullptr ? kScratchBytes : 0,
                                             static_cast<hipStream_t>(stream)));
 }

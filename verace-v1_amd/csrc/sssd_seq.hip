@@ -1,7 +1,7 @@
 // Token-sequential SSSD scan, fp32 arithmetic, one workgroup per (batch, head).
 //
-// This is the path for fp32 I/O, small problems, head_dim other than 128 and
-// the single-token decode step.  The state Psi (D x D fp32) lives in VGPRs for
+// This is the path for head_dim above 128, single tokens at head_dim other than 128, calls
+// without workspace and the sequences a chunk scan flagged as outside its accuracy envelope.  The state Psi (D x D fp32) lives in VGPRs for
 // the whole scan: thread (rg, cg) owns rows {rg + RG*m} and the four columns
 // 4cg..4cg+3, so loads and stores of Psi are float4 and fully coalesced.
 //
@@ -309,6 +309,14 @@ hipError_t launch_sssd_seq(const void* q, const void* k, const void* v, const vo
                            int io_dtype, int delta_dtype, const float* psi_in, void* out,
                            float* psi_out, int B, int T, int H, int D, hipStream_t stream,
                            const FlaggedStates& map) {
+  return launch_seq_map(q, k, v, delta, io_dtype, delta_dtype, psi_in, out, psi_out, B, T, H, D,
+                        stream, map);
+}
+
+hipError_t launch_sssd_seq(const void* q, const void* k, const void* v, const void* delta,
+                           int io_dtype, int delta_dtype, const float* psi_in, void* out,
+                           float* psi_out, int B, int T, int H, int D, hipStream_t stream,
+                           const FlaggedSegments& map) {
   return launch_seq_map(q, k, v, delta, io_dtype, delta_dtype, psi_in, out, psi_out, B, T, H, D,
                         stream, map);
 }

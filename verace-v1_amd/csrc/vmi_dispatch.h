@@ -43,6 +43,21 @@ struct FlaggedStates {
   __device__ __forceinline__ bool skip(int bh) const { return flags[bh] != tag; }
 };
 
+// Dense states, and only the sequences with a nonzero word among their nseg segments' flags run
+// (every word is written by the call's own chunk pass).
+struct FlaggedSegments {
+  static constexpr bool kSlotted = false;
+  const uint32_t* flags;  // [B * H][nseg]
+  int nseg;
+  __device__ __forceinline__ int64_t in_index(int bh, int) const { return bh; }
+  __device__ __forceinline__ int64_t out_index(int bh, int) const { return bh; }
+  __device__ __forceinline__ bool skip(int bh) const {
+    uint32_t f = 0;
+    for (int s = 0; s < nseg; ++s) f |= flags[static_cast<int64_t>(bh) * nseg + s];
+    return f == 0;
+  }
+};
+
 __device__ __forceinline__ int64_t slot_index(int s, int nslots, int bh, int H) {
   return (s >= 0 && s < nslots) ? static_cast<int64_t>(s) * H + bh % H : -1;
 }
@@ -92,6 +107,22 @@ hipError_t launch_sssd_seq(const void* q, const void* k, const void* v, const vo
                            int io_dtype, int delta_dtype, const float* psi_in, void* out,
                            float* psi_out, int B, int T, int H, int D, hipStream_t stream,
                            const FlaggedStates& map);
+hipError_t launch_sssd_seq(const void* q, const void* k, const void* v, const void* delta,
+                           int io_dtype, int delta_dtype, const float* psi_in, void* out,
+                           float* psi_out, int B, int T, int H, int D, hipStream_t stream,
+                           const FlaggedSegments& map);
+
+// sssd_chunk32.hip: chunked scan in fp32 (any I/O dtype, head_dim <= 128).
+// Below 5 tokens the token-sequential kernel is the shorter (one launch, about 4 us a token at
+// head_dim 64: 10 us at T = 2, 19.6 us at T = 5, against 16 us here for any T <= 16) and rounds no
+// more.
+constexpr int64_t kChunk32MinT = 5;
+bool use_chunk32(int64_t T, int64_t D);
+size_t chunk32_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D);
+hipError_t launch_sssd_chunk32(const void* q, const void* k, const void* v, const void* delta,
+                               int io_dtype, int delta_dtype, const float* psi_in, void* out,
+                               float* psi_out, int B, int T, int H, int D, void* workspace,
+                               hipStream_t stream);
 
 // sssd_step.hip: single-token step for head_dim 128 (persistent, two workgroups per CU,
 // heads in units of 64 columns whose loads run one unit ahead of the update and store).
@@ -117,7 +148,10 @@ hipError_t launch_sssd_step128_fused(const void* proj, int64_t proj_stride, int 
                                      const uint8_t* mask, const float* rms_w, float rms_eps,
                                      float* psi, void* out, int B, int H, hipStream_t stream);
 
-// sssd_scan.hip: picks the kernel family for a prefill scan.
+// sssd_scan.hip: picks the kernel family for a prefill scan.  scan_workspace_bytes is what the
+// fastest family uses; scan_workspace_required what a call must bring (the fp32 families run
+// token by token without any).
+size_t scan_workspace_required(int64_t B, int64_t T, int64_t H, int64_t D, int io_dtype);
 size_t scan_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D, int io_dtype);
 hipError_t dispatch_scan(const void* q, const void* k, const void* v, const void* delta,
                          int io_dtype, int delta_dtype, const float* psi_in, void* out,
