@@ -496,7 +496,7 @@ __global__ __launch_bounds__(4 * DP) void c32_pass_kernel(Args a) {
 
 // ------------------------------------------------------------------ segment start states
 // 16 columns of start_s = P_{s-1} start_{s-1} per workgroup, wave w the rows 16 w .. + 15: the
-// factor's rows come from global memory in the operand layout, the columns pass through LDS
+// factor's rows come from global memory in the operand layout two factors ahead, the columns pass through LDS
 // (transposed, so a lane's four rows are one 16-byte access); one barrier per factor.
 template <int DP>
 __global__ __launch_bounds__(4 * DP) void c32_carry_kernel(const float* __restrict__ psi_in,
@@ -516,37 +516,39 @@ __global__ __launch_bounds__(4 * DP) void c32_carry_kernel(const float* __restri
     }
     X[0][j * LU + row] = x;
   }
-  float4 p[SS];
-  auto fetch = [&](int f) {
-    const float* src = factors + ((static_cast<int64_t>(f) * BH + bh) * DP + 16 * wave + l16) * DP + 4 * g;
+  float4 pa[SS], pb[SS];
+  auto fetch = [&](float4 (&p)[SS], int f) {
+    const float* src = factors + ((static_cast<int64_t>(min(f, nf - 1)) * BH + bh) * DP + 16 * wave + l16) * DP + 4 * g;
 #pragma unroll
     for (int S = 0; S < SS; ++S) p[S] = *reinterpret_cast<const float4*>(src + 16 * S);
   };
-  fetch(0);
-  lds_barrier();
-  for (int f = 0; f < nf; ++f) {
-    const float* x = X[f & 1];
-    float4 cur[SS];
-#pragma unroll
-    for (int S = 0; S < SS; ++S) cur[S] = p[S];
-    fetch(f + 1 < nf ? f + 1 : f);
+  auto step = [&](float4 (&p)[SS], int f, int cur) {
+    const float* x = X[cur];
     f32x4 y0 = {}, y1 = {};
 #pragma unroll
     for (int S = 0; S < SS; ++S) {
       const float4 b4 = lds4(x + l16 * LU + 16 * S + 4 * g);
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
-        y0 = mma(elem(cur[S], r), elem(b4, r), y0);
-        y1 = mma(elem(cur[S], r + 1), elem(b4, r + 1), y1);
+        y0 = mma(elem(p[S], r), elem(b4, r), y0);
+        y1 = mma(elem(p[S], r + 1), elem(b4, r + 1), y1);
       }
     }
+    fetch(p, f + 2);
     const f32x4 y = y0 + y1;
-    *reinterpret_cast<float4*>(&X[(f + 1) & 1][l16 * LU + 16 * wave + 4 * g]) =
+    *reinterpret_cast<float4*>(&X[cur ^ 1][l16 * LU + 16 * wave + 4 * g]) =
         make_float4(y[0], y[1], y[2], y[3]);
     float* dst = starts + (static_cast<int64_t>(f) * BH + bh) * DP * DP + j0 + l16;
 #pragma unroll
     for (int r = 0; r < 4; ++r) dst[static_cast<int64_t>(16 * wave + 4 * g + r) * DP] = y[r];
     lds_barrier();
+  };
+  fetch(pa, 0);
+  fetch(pb, 1);
+  lds_barrier();
+  for (int f = 0; f < nf; f += 2) {
+    step(pa, f, 0);
+    if (f + 1 < nf) step(pb, f + 1, 1);
   }
 }
 
