@@ -368,6 +368,39 @@ int vmi_cham_ns_retraction(const float* h_real, const float* h_imag,
                            void* workspace, size_t workspace_bytes,
                            void* stream);
 
+/* The element-wise steps between a layer's matrix products.  dtype is the type of every tensor
+ * argument without a type of its own; rows are contiguous and 16-byte aligned, of whole 16-byte
+ * pieces (otherwise VMI_ERR_UNSUPPORTED: run the tensor operations instead).  Sums are fp32.
+ *
+ * SiTU-GLU (verace_v1/modules/activations.py:8-31): out = [beta1 tanh(gate / beta1) sigmoid(gate)]
+ * [beta2 tanh(up / beta2)], n elements. */
+int vmi_situ_glu(const void* gate, const void* up, int dtype, float beta1, float beta2, void* out,
+                 int64_t n, void* stream);
+
+/* M-CMoE coefficients (verace_v1/modules/mcmoe.py:82-117): per token, weight = softmax over the
+ * top_k of its `components` logits (ties to the lowest index), 0 elsewhere; coef[c][j] =
+ * vproj[c][j] sigmoid(sigma[c][j]) weight[c].  logits [n, components], sigma, vproj, coef
+ * [n, components, rank]; components <= 64. */
+int vmi_mcmoe_coef(const void* logits, const void* sigma, const void* vproj, int dtype, int64_t top_k,
+                   void* coef, int64_t n, int64_t components, int64_t rank, void* stream);
+
+/* x = w1 ? rmsnorm(a; w1, eps1) : a; s = (x + c) + b, rounded to dtype after each step (c, b may be
+ * NULL); stored to sum if not NULL; out = rmsnorm(s; w2, eps2) if w2 is not NULL (w2 and out together).
+ * a, b, c, sum, out [rows, d]; w1, w2 [d]. */
+int vmi_norm_add(const void* a, const void* w1, float eps1, const void* c, const void* b, void* sum,
+                 const void* w2, float eps2, void* out, int dtype, int64_t rows, int64_t d,
+                 void* stream);
+
+/* One step of the adaptive-depth loop (verace_v1/modules/acd_engine.py:128-150) for every token:
+ * out (the layer's output) and h [rows, d], w [d] and bias [1] of the halting unit and active [rows]
+ * (0 or 1) are read, h_next [rows, d] and still [rows] (the next h and active) written, final_h
+ * [rows, d], acc and depth [rows] updated in place.  mode 0: a step; 1: a step below the minimum depth
+ * (halting probability 0); 2: the loop's end, where the tokens still active add their remainder (only
+ * h, active, acc, depth and final_h are used).  threshold as rounded to dtype. */
+int vmi_halting_update(const void* out, const void* h, void* h_next, const void* w, const void* bias,
+                       void* acc, void* depth, const uint8_t* active, uint8_t* still, void* final_h,
+                       float threshold, int mode, int dtype, int64_t rows, int64_t d, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

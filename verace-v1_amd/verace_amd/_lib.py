@@ -51,6 +51,10 @@ EXPORTED = (
     "vmi_cham_step_fused",
     "vmi_cham_ns_workspace_bytes",
     "vmi_cham_ns_retraction",
+    "vmi_situ_glu",
+    "vmi_mcmoe_coef",
+    "vmi_norm_add",
+    "vmi_halting_update",
 )
 
 _lib = None
@@ -134,6 +138,16 @@ def _declare(lib):
     lib.vmi_cham_ns_workspace_bytes.restype = i32
     lib.vmi_cham_ns_retraction.argtypes = [vp, vp, vp, vp, i64, i64, i32, vp, sz, vp]
     lib.vmi_cham_ns_retraction.restype = i32
+    f32 = ctypes.c_float
+    lib.vmi_situ_glu.argtypes = [vp, vp, i32, f32, f32, vp, i64, vp]
+    lib.vmi_situ_glu.restype = i32
+    lib.vmi_mcmoe_coef.argtypes = [vp, vp, vp, i32, i64, vp, i64, i64, i64, vp]
+    lib.vmi_mcmoe_coef.restype = i32
+    lib.vmi_norm_add.argtypes = [vp, vp, f32, vp, vp, vp, vp, f32, vp, i32, i64, i64, vp]
+    lib.vmi_norm_add.restype = i32
+    lib.vmi_halting_update.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, f32, i32, i32, i64, i64,
+                                       vp]
+    lib.vmi_halting_update.restype = i32
 
 
 def load(path: str = LIB_PATH):

@@ -38,6 +38,7 @@ import torch.nn as nn
 
 from .cham_memory import ContinuousHolographicMemory
 from .hip_kernels import newton_schulz_unitary_retraction
+from .layer_ops import HaltingState, norm_add, plain
 from .mcmoe import ManifoldContinuousMoE
 from .sssd_attention import SSSDAttention
 
@@ -92,22 +93,38 @@ class VeraceV1Layer(nn.Module):
             block_residual = torch.cat([block_residual, flat_h.unsqueeze(1)], dim=1)
         sssd_out, new_sssd_state = self.sssd_attn(self.sssd_norm(h_in), initial_state=sssd_state,
                                                   return_state=True, active_mask=active_mask)
-        h_mid1 = h_in + sssd_out
-        cham_out, new_holo = self.cham_memory(self.cham_norm(h_mid1), initial_hologram=cham_hologram,
-                                              active_mask=active_mask)
-        h_mid2 = h_mid1 + cham_out
-        h_out = h_mid2 + self.mcmoe(self.mcmoe_norm(h_mid2))
-        return h_out, block_residual, new_sssd_state, new_holo
+        h_mid1, x = norm_add(sssd_out, b=h_in, norm2=self.cham_norm)
+        if plain(self.cham_memory, ContinuousHolographicMemory):
+            # the memory's own norm joins the residual add and the next norm
+            y, new_holo = self.cham_memory.before_norm(x, cham_hologram, active_mask)
+            h_mid2, x = norm_add(y, self.cham_memory.norm, b=h_mid1, norm2=self.mcmoe_norm)
+        else:
+            y, new_holo = self.cham_memory(x, initial_hologram=cham_hologram, active_mask=active_mask)
+            h_mid2, x = norm_add(y, b=h_mid1, norm2=self.mcmoe_norm)
+        return self._mcmoe_residual(h_mid2, x), block_residual, new_sssd_state, new_holo
+
+    def _mcmoe_residual(self, h: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+        """h + mcmoe(x)."""
+        if plain(self.mcmoe, ManifoldContinuousMoE):
+            base_out, adapt = self.mcmoe.parts(x)
+            return norm_add(adapt, self.mcmoe.norm, base_out, h.reshape(adapt.shape))[0].view(h.shape)
+        return h + self.mcmoe(x)
 
     def step_(self, h_in: torch.Tensor, st: "LayerDecodeState",
               active_mask: Optional[torch.Tensor] = None) -> torch.Tensor:
         """One token per item (h_in [B, 1, hidden]) with this layer's states updated in
         place; the same sub-layers as :meth:`forward` (no block residual: a decode call's
         layers never receive a snapshot, see the module docstring)."""
-        h_mid1 = h_in + self.sssd_attn.step_(self.sssd_norm(h_in), st.sssd, active_mask)
-        cham_out = self.cham_memory.step_(self.cham_norm(h_mid1), st.cham, st.cham_readout, active_mask)
-        h_mid2 = h_mid1 + cham_out
-        return h_mid2 + self.mcmoe(self.mcmoe_norm(h_mid2))
+        h_mid1, x = norm_add(self.sssd_attn.step_(self.sssd_norm(h_in), st.sssd, active_mask), b=h_in,
+                             norm2=self.cham_norm)
+        cm = self.cham_memory
+        if type(cm) is ContinuousHolographicMemory and "step_" not in cm.__dict__:
+            y = cm.step_before_norm_(x, st.cham, st.cham_readout, active_mask)
+            h_mid2, x = norm_add(y, cm.norm, b=h_mid1, norm2=self.mcmoe_norm)
+        else:
+            h_mid2, x = norm_add(cm.step_(x, st.cham, st.cham_readout, active_mask), b=h_mid1,
+                                 norm2=self.mcmoe_norm)
+        return self._mcmoe_residual(h_mid2, x)
 
 
 class AdaptiveCognitiveDepthEngine(nn.Module):
@@ -140,6 +157,10 @@ class AdaptiveCognitiveDepthEngine(nn.Module):
         depth = torch.zeros(b, s, device=h_in.device, dtype=h_in.dtype)
         active = torch.ones(b, s, device=h_in.device, dtype=torch.bool)
         n_layers = min(len(layers), max_depth)
+        fused = None
+        if (type(self) is AdaptiveCognitiveDepthEngine
+                and "compute_halting_probability" not in self.__dict__):
+            fused = HaltingState.start(self.w_halting, self.energy_threshold, h_curr, final_h, acc, depth)
         states_out = None
         if step_states is None:
             states_out = [(list(initial_layer_states[l]) if initial_layer_states is not None
@@ -149,16 +170,20 @@ class AdaptiveCognitiveDepthEngine(nn.Module):
             if not static_control and not bool(active.any()):
                 break
             layer = layers[l_idx]
-            item_on = active.any(dim=1)                              # items with work here
             mask = active if static_control or not bool(active.all()) else None
             if step_states is not None:
                 out = layer.step_(h_curr, step_states.layers[l_idx], mask)
             else:
+                item_on = active.any(dim=1)                          # items with work here
                 sst, holo = _stack_states(states_out[l_idx], item_on, layer, h_in)
                 out, _, new_s, new_h = layer(h_curr, sssd_state=sst, cham_hologram=holo, active_mask=mask)
                 for i in range(b):
                     if bool(item_on[i]):
                         states_out[l_idx][i] = (new_s[i:i + 1], (new_h[0][i:i + 1], new_h[1][i:i + 1]))
+            if fused is not None and fused.accepts(out, h_curr):  # the lines below in one kernel
+                h_curr, active = fused.step(out, h_curr, active, l_idx < min_depth)
+                continue
+            fused = None
             h_next = torch.where(active.unsqueeze(-1), out, h_curr)
             p = self.compute_halting_probability(h_next)
             if l_idx < min_depth:
@@ -176,6 +201,9 @@ class AdaptiveCognitiveDepthEngine(nn.Module):
             active = still
             h_curr = h_next
         if static_control or bool(active.any()):
+            if fused is not None:
+                fused.finish(h_curr, active)
+                return final_h, depth, states_out
             rem = (1.0 - acc).clamp(min=0.0)
             final_h = final_h + (rem * active.to(h_in.dtype)).unsqueeze(-1) * h_curr
             depth = depth + rem * active.to(h_in.dtype)

@@ -89,6 +89,11 @@ class ContinuousHolographicMemory(nn.Module):
         initial_hologram: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
         active_mask: Optional[torch.Tensor] = None,
     ) -> Tuple[torch.Tensor, Tuple[torch.Tensor, torch.Tensor]]:
+        y, hologram = self.before_norm(x, initial_hologram, active_mask)
+        return self.norm(y), hologram
+
+    def before_norm(self, x, initial_hologram=None, active_mask=None):
+        """:meth:`forward` without its last step, the RMSNorm."""
         if not x.is_cuda:
             raise RuntimeError("verace_amd.ContinuousHolographicMemory runs on a HIP device only")
         if torch.is_grad_enabled() and x.requires_grad:
@@ -101,8 +106,7 @@ class ContinuousHolographicMemory(nn.Module):
         else:
             q, k, v, gamma = self.project(x, active_mask)
             rec, hologram = launch_cham_hip_update(q, k, v, gamma, initial_hologram)
-        y = self.norm(self.w_out(rec.to(self.w_out.weight.dtype)))
-        return y, hologram
+        return self.w_out(rec.to(self.w_out.weight.dtype)), hologram
 
     def step_(self, x: torch.Tensor, hologram: Tuple[torch.Tensor, torch.Tensor],
               readout: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
@@ -111,10 +115,14 @@ class ContinuousHolographicMemory(nn.Module):
         [B, h, h] float32 updated in place.  ``readout`` is the readout state
         R = NS_3(H) carried beside H (updated in place too) when H is not unitary; None
         when H came from the identity start (then NS_3(H) = H).  Returns y [B, 1, hidden]."""
+        return self.norm(self.step_before_norm_(x, hologram, readout, active_mask))
+
+    def step_before_norm_(self, x, hologram, readout=None, active_mask=None):
+        """:meth:`step_` without its last step, the RMSNorm."""
         if self._fused_step(x):  # one projection GEMM; normalisation and gamma in the kernel
             rec = cham_step_fused_(F.linear(x, self._stacked_weight()), self.holographic_dim,
                                    hologram, readout, active_mask)
         else:
             q, k, v, gamma = self.project(x, active_mask)
             rec = cham_step_(q, k, v, gamma, hologram, readout)
-        return self.norm(self.w_out(rec.to(self.w_out.weight.dtype)))
+        return self.w_out(rec.to(self.w_out.weight.dtype))

@@ -36,6 +36,13 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _mask_bytes(mask: torch.Tensor) -> torch.Tensor:
+    """An active mask as contiguous bytes (nonzero = active); a bool tensor's own bytes as they are."""
+    if mask.dtype == torch.bool:
+        return mask.contiguous().view(torch.uint8)
+    return mask.to(torch.uint8).contiguous()
+
+
 def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
@@ -250,7 +257,7 @@ def launch_sssd_hip_scan_fused(
     mask = None
     if active_mask is not None:
         _require_device(active_mask, "active_mask")
-        mask = active_mask.reshape(b, s).to(torch.uint8).contiguous()
+        mask = _mask_bytes(active_mask.reshape(b, s))
     w = None
     eps = 0.0
     if rms_weight is not None:
@@ -357,7 +364,7 @@ def sssd_step_fused_(
     mask = None
     if active_mask is not None:
         _require_device(active_mask, "active_mask")
-        mask = active_mask.reshape(b).to(torch.uint8).contiguous()
+        mask = _mask_bytes(active_mask.reshape(b))
     w = None
     eps = 0.0
     if rms_weight is not None:
@@ -466,7 +473,7 @@ def launch_cham_hip_update_fused(
     mask = None
     if active_mask is not None:
         _require_device(active_mask, "active_mask")
-        mask = active_mask.reshape(b, s).to(torch.uint8).contiguous()
+        mask = _mask_bytes(active_mask.reshape(b, s))
     out = _aligned(torch.empty(b, s, h, device=proj.device, dtype=proj.dtype))
     hr = torch.empty(b, h, h, device=proj.device, dtype=torch.float32)
     hi = torch.empty(b, h, h, device=proj.device, dtype=torch.float32)
@@ -525,7 +532,7 @@ def cham_step_fused_(
     mask = None
     if active_mask is not None:
         _require_device(active_mask, "active_mask")
-        mask = active_mask.reshape(B).to(torch.uint8).contiguous()
+        mask = _mask_bytes(active_mask.reshape(B))
     out = torch.empty(B, 1, h, device=proj.device, dtype=proj.dtype)
     lib = _lib.load()
     ws_bytes = ctypes.c_size_t(0)

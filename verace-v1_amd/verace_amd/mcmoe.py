@@ -1,5 +1,6 @@
-"""The layer's third sub-block, M-CMoE, as torch ops (not on the accelerated path; the layer
-harness needs it to run the reference's layer).
+"""The layer's third sub-block, M-CMoE: library GEMMs with the steps between them (activation,
+routing coefficients, norm and adds) on the fused kernels of :mod:`verace_amd.layer_ops` in
+inference, as torch ops otherwise.
 
 ``SiTUGLU`` restates ``verace_v1/modules/activations.py:8-31`` and
 ``ManifoldContinuousMoE`` restates ``verace_v1/modules/mcmoe.py:20-120`` with the same
@@ -14,6 +15,8 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+
+from .layer_ops import mcmoe_coef, norm_add, situ_glu
 
 
 class SiTUGLU(nn.Module):
@@ -32,8 +35,7 @@ class SiTUGLU(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         g = self.w_gate(x)
         u = self.w_up(x)
-        return (self.beta1 * torch.tanh(g / self.beta1) * torch.sigmoid(g)) * \
-            (self.beta2 * torch.tanh(u / self.beta2))
+        return situ_glu(g, u, self.beta1, self.beta2)
 
 
 class ManifoldContinuousMoE(nn.Module):
@@ -52,20 +54,18 @@ class ManifoldContinuousMoE(nn.Module):
         self.hyper_sigma = nn.Linear(hidden_dim, num_components * rank, bias=False)
         self.norm = nn.RMSNorm(hidden_dim)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def parts(self, x: torch.Tensor):
+        """The base path and the manifold path before its norm, both [tokens, hidden]."""
         b, s, d = x.shape
         C, r = self.num_components, self.rank
         xf = x.reshape(b * s, d)
         base_out = self.base_w_down(self.base_situ_glu(xf))
-        # keep-top-k before the softmax (mcmoe.py:82-87)
-        kv = min(self.top_k_components, C)
-        logits = self.router(xf)
-        top_l, top_i = torch.topk(logits, k=kv, dim=-1)
-        masked = torch.full_like(logits, float("-inf")).scatter(-1, top_i, top_l)
-        weights = torch.softmax(masked, dim=-1)                   # exactly 0 off the top k
-        sigma = torch.sigmoid(self.hyper_sigma(xf)).view(b * s, C, r)
         # v_proj[n, j, :] = V_j x_n for every component, then the selected ones' coefficients
-        vproj = (xf @ self.v_basis.reshape(C * r, d).t()).view(b * s, C, r)
-        coef = (vproj * sigma * weights.unsqueeze(-1)).reshape(b * s, C * r)
-        adapt = coef @ self.u_basis.permute(0, 2, 1).reshape(C * r, d)
-        return (base_out + self.norm(adapt)).view(b, s, d)
+        vproj = xf @ self.v_basis.reshape(C * r, d).t()
+        coef = mcmoe_coef(self.router(xf), self.hyper_sigma(xf), vproj, min(self.top_k_components, C))
+        return base_out, coef @ self.u_basis.permute(0, 2, 1).reshape(C * r, d)
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        b, s, d = x.shape
+        base_out, adapt = self.parts(x)
+        return norm_add(adapt, self.norm, base_out)[0].view(b, s, d)
