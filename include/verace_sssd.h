@@ -368,6 +368,15 @@ int vmi_cham_ns_retraction(const float* h_real, const float* h_imag,
                            void* workspace, size_t workspace_bytes,
                            void* stream);
 
+/* L2 normalisation of rows and its gradient (F.normalize over the last dimension, as
+ * verace_v1/modules/sssd_attention.py:116-119 applies it to q, k, v): y = x / max(|x|, eps);
+ * dx = (dy - y (y . dy)) / |x| for |x| >= eps, dy / eps below.  x, dx [rows, D] x_dtype, y, dy [rows, D]
+ * y_dtype; the types are equal (F32 or BF16) or y is F32.  D <= 1024. */
+int vmi_unit_rows(const void* x, int x_dtype, void* y, int y_dtype, int64_t rows, int64_t D, float eps,
+                  void* stream);
+int vmi_unit_rows_bwd(const void* x, int x_dtype, const void* dy, int y_dtype, void* dx, int64_t rows,
+                      int64_t D, float eps, void* stream);
+
 /* The element-wise steps between a layer's matrix products.  dtype is the type of every tensor
  * argument without a type of its own; rows are contiguous and 16-byte aligned, of whole 16-byte
  * pieces (otherwise VMI_ERR_UNSUPPORTED: run the tensor operations instead).  Sums are fp32.

@@ -51,6 +51,8 @@ EXPORTED = (
     "vmi_cham_step_fused",
     "vmi_cham_ns_workspace_bytes",
     "vmi_cham_ns_retraction",
+    "vmi_unit_rows",
+    "vmi_unit_rows_bwd",
     "vmi_situ_glu",
     "vmi_mcmoe_coef",
     "vmi_norm_add",
@@ -139,6 +141,10 @@ def _declare(lib):
     lib.vmi_cham_ns_retraction.argtypes = [vp, vp, vp, vp, i64, i64, i32, vp, sz, vp]
     lib.vmi_cham_ns_retraction.restype = i32
     f32 = ctypes.c_float
+    lib.vmi_unit_rows.argtypes = [vp, i32, vp, i32, i64, i64, f32, vp]
+    lib.vmi_unit_rows.restype = i32
+    lib.vmi_unit_rows_bwd.argtypes = [vp, i32, vp, i32, vp, i64, i64, f32, vp]
+    lib.vmi_unit_rows_bwd.restype = i32
     lib.vmi_situ_glu.argtypes = [vp, vp, i32, f32, f32, vp, i64, vp]
     lib.vmi_situ_glu.restype = i32
     lib.vmi_mcmoe_coef.argtypes = [vp, vp, vp, i32, i64, vp, i64, i64, i64, vp]

@@ -193,6 +193,56 @@ class SSSDScanFunction(torch.autograd.Function):
                 None if dpsi0 is None else dpsi0.to(ctx.init_dtype))
 
 
+_UNIT_EPS = 1e-12  # F.normalize's default
+
+
+class UnitRowsFunction(torch.autograd.Function):
+    """``F.normalize(x, dim=-1)`` of contiguous rows in one kernel each way; the result in
+    ``out_dtype``.  A backward that is itself differentiated runs the torch ops."""
+
+    @staticmethod
+    def forward(ctx, x, out_dtype):
+        y = torch.empty(x.shape, device=x.device, dtype=out_dtype)
+        D = x.shape[-1]
+        _lib.check(_lib.load().vmi_unit_rows(_ptr(x), _lib.dtype_code(x.dtype), _ptr(y),
+                                             _lib.dtype_code(out_dtype), x.numel() // D, D, _UNIT_EPS,
+                                             _lib.stream_handle(x.device)), "vmi_unit_rows")
+        ctx.save_for_backward(x)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, = ctx.saved_tensors
+        if torch.is_grad_enabled():  # create_graph
+            with torch.autocast("cuda", enabled=False):
+                n = torch.linalg.vector_norm(x.to(dy.dtype), dim=-1, keepdim=True).clamp_min(_UNIT_EPS)
+                y = x.to(dy.dtype) / n
+                return ((dy - y * (y * dy).sum(-1, keepdim=True)) / n).to(x.dtype), None
+        dy = dy.contiguous()
+        dx = torch.empty_like(x)
+        D = x.shape[-1]
+        _lib.check(_lib.load().vmi_unit_rows_bwd(_ptr(x), _lib.dtype_code(x.dtype), _ptr(dy),
+                                                 _lib.dtype_code(dy.dtype), _ptr(dx), x.numel() // D, D,
+                                                 _UNIT_EPS, _lib.stream_handle(x.device)),
+                   "vmi_unit_rows_bwd")
+        return dx, None
+
+
+def unit_rows(x: torch.Tensor) -> torch.Tensor:
+    """``F.normalize(x, p=2, dim=-1)``, on the fused kernels for plain device tensors that autograd
+    differentiates.  Under autocast the result of 16-bit rows is fp32, as F.normalize's; fp16 rows
+    without autocast keep its op sequence (there eps rounds to zero)."""
+    out = torch.float32 if torch.is_autocast_enabled("cuda") else x.dtype
+    if (type(x) is torch.Tensor and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and (x.dtype, out) != (torch.float16, torch.float16) and 1 <= x.shape[-1] <= 1024
+            and 0 < x.numel() // x.shape[-1] < 2 ** 31 and x.is_contiguous()
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0):
+        return UnitRowsFunction.apply(x, out)
+    return torch.nn.functional.normalize(x, p=2, dim=-1)
+
+
 def sssd_scan(q, k, v, delta, initial_state=None):
     """:func:`launch_sssd_hip_scan`, differentiable when autograd needs it."""
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad

@@ -20,6 +20,7 @@ on the HIP backward kernels.
 """
 from __future__ import annotations
 
+from functools import partial
 from typing import Optional, Tuple
 
 import torch
@@ -28,7 +29,8 @@ import torch.nn.functional as F
 
 from . import ops as _ops  # noqa: F401  (registers torch.ops.verace.*)
 from .hip_kernels import (fused_scan_supported, fused_step_supported, launch_sssd_hip_scan,
-                          launch_sssd_hip_scan_fused, sssd_scan, sssd_step_, sssd_step_fused_)
+                          launch_sssd_hip_scan_fused, sssd_scan, sssd_step_, sssd_step_fused_,
+                          unit_rows)
 
 
 def _traced(x: torch.Tensor) -> bool:
@@ -92,14 +94,13 @@ class SSSDAttention(nn.Module):
         return launch_sssd_hip_scan_fused(proj, self.num_heads, self.head_dim, active_mask,
                                           w.detach(), self.head_rmsnorm.eps, initial_state)
 
-    def project(self, x: torch.Tensor, active_mask: Optional[torch.Tensor] = None):
-        """q, k, v [B,T,H,D] (L2-normalised) and delta [B,T,H] as the reference builds them
-        (``sssd_attention.py:116-126``)."""
+    def project(self, x: torch.Tensor, active_mask: Optional[torch.Tensor] = None,
+                norm=partial(F.normalize, p=2, dim=-1)):
+        """q, k, v [B,T,H,D] (L2-normalised, by ``norm``) and delta [B,T,H] as the reference builds
+        them (``sssd_attention.py:116-126``)."""
         b, s, _ = x.shape
         H, D = self.num_heads, self.head_dim
-        q = F.normalize(self.w_q(x).view(b, s, H, D), p=2, dim=-1)
-        k = F.normalize(self.w_k(x).view(b, s, H, D), p=2, dim=-1)
-        v = F.normalize(self.w_v(x).view(b, s, H, D), p=2, dim=-1)
+        q, k, v = (norm(w(x).view(b, s, H, D)) for w in (self.w_q, self.w_k, self.w_v))
         delta = 0.1 * torch.sigmoid(self.w_delta(x)).view(b, s, H, 1)
         if active_mask is not None:
             while active_mask.ndim < delta.ndim:
@@ -130,7 +131,7 @@ class SSSDAttention(nn.Module):
         rms_grad = (torch.is_grad_enabled() and self.head_rmsnorm.weight is not None
                     and self.head_rmsnorm.weight.requires_grad)
         if grad:
-            q, k, v, delta = self.project(x, active_mask)
+            q, k, v, delta = self.project(x, active_mask, unit_rows)
             o, psi = sssd_scan(q, k, v, delta, initial_state)
             o_norm = self.head_rmsnorm(o).view(b, s, self.num_heads * self.head_dim)
         elif self._fused(x):
