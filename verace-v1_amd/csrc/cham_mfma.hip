@@ -12,7 +12,7 @@
 //
 // Launches (before the readout kernels of cham_wide.hip, which read the snapshots written
 // here exactly as they read the token-sequential kernel's):
-//   1. cm_prep_kernel, one wave per (chunk, sequence): k, v converted to f16 (non-finite
+//   1. cm_prep_kernel, one workgroup per (chunk, sequence): k, v converted to f16 (non-finite
 //      elements zeroed) and stored in the column kernel's MFMA operand layout (each
 //      16-feature block of the chunk's 32 rank rows as 64 lanes x 16 bytes, so every operand
 //      load is a contiguous 1 KB), G on the MFMA from them, then T by
@@ -141,16 +141,21 @@ __device__ __forceinline__ void split8p(const float* x, V8& hi, V8& lo) {
 // elements: k at h, v at 2h), v through silu, both scaled by the norms the fused coefficient
 // kernel stored (coef floats 6 and 7) and rounded by cham::fused_f16, as that kernel did for
 // the Gram entries of its coefficients.
+// PWV waves share a chunk: wave w converts every PWV-th 16-feature block (four in flight) and sums
+// its part of G; one wave then solves for T, all write it out.  (One wave per chunk left half the
+// SIMDs idle at B4 T2048 and ran its 64 blocks one load after the other: 67 us fused there, 32 now.)
+constexpr int PWV = 8;
 template <typename IO, bool FUSED = false>
-__global__ __launch_bounds__(64) void cm_prep_kernel(const IO* __restrict__ k,
-                                                     const IO* __restrict__ v,
-                                                     const float* __restrict__ coef,
-                                                     E* __restrict__ tt, E* __restrict__ yop,
-                                                     int T, int h, int hp, int64_t stride = 0) {
+__global__ __launch_bounds__(64 * PWV) void cm_prep_kernel(const IO* __restrict__ k,
+                                                           const IO* __restrict__ v,
+                                                           const float* __restrict__ coef,
+                                                           E* __restrict__ tt, E* __restrict__ yop,
+                                                           int T, int h, int hp, int64_t stride = 0) {
+  __shared__ float Gp[PWV][RK][RK + 1];
   __shared__ float G[RK][RK + 1];
   __shared__ float Nc[CT][NCF];
   __shared__ float Tf[2][RK][RK + 1];
-  const int lane = threadIdx.x, l32 = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int m = blockIdx.x, b = blockIdx.y, nc = gridDim.x;
   const int t0 = m * CT;
   // Gram: lane (rho = l32, g) holds features 16 ks + 8 g + 0..7 of rank row rho
@@ -159,51 +164,69 @@ __global__ __launch_bounds__(64) void cm_prep_kernel(const IO* __restrict__ k,
   const int64_t row = static_cast<int64_t>(b) * T + (tok_ok ? tok : 0);
   const IO* src = FUSED ? k + row * stride + ((l32 & 1) ? 2 * h : h) : ((l32 & 1) ? v : k) + row * h;
   const float scale = FUSED ? coef[row * NCF + 6 + (l32 & 1)] : 1.f;
+  for (int e = tid; e < CT * NCF; e += 64 * PWV) {
+    const int t = e / NCF;
+    Nc[t][e % NCF] = t0 + t < T ? coef[(static_cast<int64_t>(b) * T + t0 + t) * NCF + e % NCF] : 0.f;
+  }
   // operand block kb of this chunk: lane (rho, g) holds features 16 kb + 4 g + {0..3} and
   // 16 kb + 8 + 4 g + {0..3} of rank row rho (the K order of the column kernel's state tiles;
   // G sums over every feature, so any order serves it); blocks past h and tokens past T are 0
   E* dst = yop + (static_cast<int64_t>(b) * nc + m) * (hp / 16) * 512 + lane * 8;
   f32x16 acc = {};
-  const int nks = (h + 15) / 16;  // the same trip counts in both half-waves (MFMA is wave-wide)
-  for (int ks = 0; ks < hp / 16; ++ks) {
-    const int f0 = 16 * ks + 4 * g, f1 = f0 + 8;  // h % 4 == 0: a piece is wholly in or out
-    uint2 r0 = make_uint2(0, 0), r1 = make_uint2(0, 0);
-    if (tok_ok && f0 < h) r0 = *reinterpret_cast<const uint2*>(src + f0);
-    if (tok_ok && f1 < h) r1 = *reinterpret_cast<const uint2*>(src + f1);
-    V8 x;
-    if constexpr (FUSED) {
-      float f[8];
-      unpack4<IO>(r0, f);
-      unpack4<IO>(r1, f + 4);
+  constexpr int NB = 4;  // blocks whose loads a wave has in flight
+  for (int k0 = wave; k0 < hp / 16; k0 += PWV * NB) {  // the same trip counts in both half-waves
+    uint2 r0[NB], r1[NB];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float y = (l32 & 1) ? cham::silu_f(f[i]) : f[i];
-        x[i] = cham::fused_f16(y, scale);
-      }
-      if (!(tok_ok && f0 < h)) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = static_cast<E>(0.f);
-      }
-      if (!(tok_ok && f1 < h)) {
-#pragma unroll
-        for (int i = 4; i < 8; ++i) x[i] = static_cast<E>(0.f);
-      }
-    } else {
-      x = cat8<V4, V8>(to_f16x4<IO>(r0, true), to_f16x4<IO>(r1, true));
+    for (int u = 0; u < NB; ++u) {
+      const int f0 = 16 * (k0 + PWV * u) + 4 * g, f1 = f0 + 8;  // h % 4 == 0: a piece is wholly in or out
+      r0[u] = *reinterpret_cast<const uint2*>(src + (f0 < h ? f0 : 0));
+      r1[u] = *reinterpret_cast<const uint2*>(src + (f1 < h ? f1 : 0));
+      if (!tok_ok || f0 >= h) r0[u] = make_uint2(0, 0);
+      if (!tok_ok || f1 >= h) r1[u] = make_uint2(0, 0);
     }
-    *reinterpret_cast<V8*>(dst + ks * 512) = x;
-    if (ks < nks) acc = MM::mma32(x, x, acc);
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int ks = k0 + PWV * u;
+      if (ks >= hp / 16) break;
+      V8 x;
+      if constexpr (FUSED) {
+        const int f0 = 16 * ks + 4 * g, f1 = f0 + 8;
+        float f[8];
+        unpack4<IO>(r0[u], f);
+        unpack4<IO>(r1[u], f + 4);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float y = (l32 & 1) ? cham::silu_f(f[i]) : f[i];
+          x[i] = cham::fused_f16(y, scale);
+        }
+        if (!(tok_ok && f0 < h)) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] = static_cast<E>(0.f);
+        }
+        if (!(tok_ok && f1 < h)) {
+#pragma unroll
+          for (int i = 4; i < 8; ++i) x[i] = static_cast<E>(0.f);
+        }
+      } else {
+        x = cat8<V4, V8>(to_f16x4<IO>(r0[u], true), to_f16x4<IO>(r1[u], true));
+      }
+      *reinterpret_cast<V8*>(dst + ks * 512) = x;
+      acc = MM::mma32(x, x, acc);
+    }
   }
 #pragma unroll
-  for (int r = 0; r < 16; ++r) G[8 * (r >> 2) + 4 * g + (r & 3)][l32] = acc[r];
-  for (int e = lane; e < CT * NCF; e += 64) {
-    const int t = e / NCF;
-    Nc[t][e % NCF] = t0 + t < T ? coef[(static_cast<int64_t>(b) * T + t0 + t) * NCF + e % NCF] : 0.f;
+  for (int r = 0; r < 16; ++r) Gp[wave][8 * (r >> 2) + 4 * g + (r & 3)][l32] = acc[r];
+  __syncthreads();
+  for (int e = tid; e < RK * RK; e += 64 * PWV) {
+    float x = 0.f;
+#pragma unroll
+    for (int w = 0; w < PWV; ++w) x += Gp[w][e / RK][e % RK];
+    G[e / RK][e % RK] = x;
   }
   __syncthreads();
   // T = (I - L)^-1 blockdiag(N): block row t = N_t (E_t + sum_{i<t} G_ti T_i); lane j < 32
   // computes column j (rows 0 .. 31, complex)
-  if (lane < RK) {
+  if (tid < RK) {
     const int j = lane;
     float xr[RK], xi[RK];
 #pragma unroll
@@ -231,23 +254,19 @@ __global__ __launch_bounds__(64) void cm_prep_kernel(const IO* __restrict__ k,
     }
   }
   __syncthreads();
-  // row-major hi / lo parts: lane = (part, row) writes the row's 32 values
-  {
-    const int part = lane >> 5, row = lane & 31;
-    E* dh = tt + (static_cast<int64_t>(b) * nc + m) * TT_STRIDE + (2 * part) * RK * RK + row * RK;
-    E* dl = dh + RK * RK;
+  // row-major hi / lo parts, eight consecutive values of a row per thread
+  if (tid < 2 * RK * RK / 8) {
+    const int part = tid / (RK * RK / 8), e = 8 * (tid % (RK * RK / 8)), rr = e / RK, c0 = e % RK;
+    E* dh = tt + (static_cast<int64_t>(b) * nc + m) * TT_STRIDE + (2 * part) * RK * RK + e;
+    V8 hi, lo;
 #pragma unroll
-    for (int q = 0; q < RK / 8; ++q) {
-      V8 hi, lo;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float x = TSCALE * Tf[part][row][8 * q + i];
-        hi[i] = static_cast<E>(x);
-        lo[i] = static_cast<E>(x - static_cast<float>(hi[i]));
-      }
-      *reinterpret_cast<V8*>(dh + 8 * q) = hi;
-      *reinterpret_cast<V8*>(dl + 8 * q) = lo;
+    for (int i = 0; i < 8; ++i) {
+      const float x = TSCALE * Tf[part][rr][c0 + i];
+      hi[i] = static_cast<E>(x);
+      lo[i] = static_cast<E>(x - static_cast<float>(hi[i]));
     }
+    *reinterpret_cast<V8*>(dh) = hi;
+    *reinterpret_cast<V8*>(dh + RK * RK) = lo;
   }
 }
 
@@ -265,6 +284,41 @@ struct alignas(16) ColsSmem {
   E zl[32][Z_LD];
   E yt[NWV][RK][Y_LD];
 };
+
+// A plane's 16 columns c0 .. c0 + 15 (row-major [h][h]) as 16-byte pieces, piece e = tid + NTH u
+// holding columns c0 + 4 (e % 4) .. + 3 of row e / 4 (zeros past h): every load of the thread in
+// flight at once, and LDS rows of 20 floats.  (4-byte loads in a loop, each stored to a column-major
+// tile 16 banks apart, took 47 us of a call's start and end at B4 h1024, so about 22.)
+constexpr int TILE_LD = COLS + 4;
+__device__ __forceinline__ bool planes_vec(int h, const float* a, const float* b) {
+  return h % 4 == 0 && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) % 16) == 0;
+}
+template <int PV>
+__device__ __forceinline__ void load_plane(const float* __restrict__ src, int h, int c0, int tid,
+                                           bool vec, float4 (&x)[PV]) {
+  if (vec) {
+#pragma unroll
+    for (int u = 0; u < PV; ++u) {
+      const int e = tid + NTH * u, r = e / 4, cc = c0 + 4 * (e % 4);
+      x[u] = *reinterpret_cast<const float4*>(src + static_cast<int64_t>(min(r, h - 1)) * h + min(cc, h - 4));
+    }
+#pragma unroll
+    for (int u = 0; u < PV; ++u) {
+      const int e = tid + NTH * u;
+      if (e / 4 >= h || c0 + 4 * (e % 4) >= h) x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < PV; ++u) {
+      const int e = tid + NTH * u, r = e / 4, cc = c0 + 4 * (e % 4);
+      const float* p = src + static_cast<int64_t>(r) * h;
+      x[u].x = r < h && cc < h ? p[cc] : 0.f;
+      x[u].y = r < h && cc + 1 < h ? p[cc + 1] : 0.f;
+      x[u].z = r < h && cc + 2 < h ? p[cc + 2] : 0.f;
+      x[u].w = r < h && cc + 3 < h ? p[cc + 3] : 0.f;
+    }
+  }
+}
 
 // Workgroup (column block cb, sequence b, state z).  Lane (n = lane % 32, g = lane / 32)
 // of wave w holds, in tile rt, rows w RPW + 32 rt + 8 (r/4) + 4 g + r%4 of MFMA column n:
@@ -301,38 +355,44 @@ __global__ __launch_bounds__(NTH) void cm_cols_kernel(
   {
     const float* ir = z == 0 ? i0r : i1r;
     const float* ii = z == 0 ? i0i : i1i;
-    float* tile = &sm.wpart[0][0][0];  // [COLS][HP] floats of one plane (<= 64 KB)
-    static_assert(sizeof(ColsSmem<TPW>) >= sizeof(float) * COLS * HP, "tile does not fit");
+    // [rows][COLS] of one plane; both planes' loads are issued before the first wait
+    float* tile = &sm.wpart[0][0][0];
+    static_assert(sizeof(ColsSmem<TPW>) >= sizeof(float) * TILE_LD * HP, "tile does not fit");
+    constexpr int PV = HP * COLS / 4 / NTH;  // 16-byte pieces per thread and plane
+    const bool vec = planes_vec(h, ir, ii);
+    float4 pr[PV], pi[PV];
+    if (ir) load_plane<PV>(ir + b * hh, h, c0, tid, vec, pr);
+    if (ii) load_plane<PV>(ii + b * hh, h, c0, tid, vec, pi);
 #pragma unroll
     for (int rt = 0; rt < TPW; ++rt) hs[rt] = f32x16{};
-    for (int p = 0; p < 2; ++p) {
-      const float* src = p == 0 ? ir : ii;
-      if (src) {
-        for (int e = tid; e < h * COLS; e += NTH) {
-          const int r = e / COLS, cc = e % COLS;
-          tile[cc * HP + r] = c0 + cc < h ? src[b * hh + static_cast<int64_t>(r) * h + c0 + cc] : 0.f;
-        }
-        __syncthreads();
-        if (part == p) {
+    auto take = [&](const float4 (&x)[PV], int p) {
 #pragma unroll
-          for (int rt = 0; rt < TPW; ++rt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int row = r0w + 32 * rt + 8 * (r >> 2) + 4 * g + (r & 3);
-              hs[rt][r] = row < h ? tile[ncol * HP + row] : 0.f;
-            }
-        }
-        __syncthreads();
-      } else if (p == 0) {  // identity
+      for (int u = 0; u < PV; ++u) {
+        const int e = tid + NTH * u;
+        *reinterpret_cast<float4*>(tile + (e / 4) * TILE_LD + 4 * (e % 4)) = x[u];
+      }
+      __syncthreads();
+      if (part == p) {
 #pragma unroll
         for (int rt = 0; rt < TPW; ++rt)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = r0w + 32 * rt + 8 * (r >> 2) + 4 * g + (r & 3);
-            hs[rt][r] = (part == 0 && colok && row == col) ? 1.f : 0.f;
-          }
+          for (int r = 0; r < 16; ++r)
+            hs[rt][r] = tile[(r0w + 32 * rt + 8 * (r >> 2) + 4 * g + (r & 3)) * TILE_LD + ncol];
       }
+      __syncthreads();
+    };
+    if (ir) {
+      take(pr, 0);
+    } else {  // identity
+#pragma unroll
+      for (int rt = 0; rt < TPW; ++rt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = r0w + 32 * rt + 8 * (r >> 2) + 4 * g + (r & 3);
+          hs[rt][r] = (part == 0 && colok && row == col) ? 1.f : 0.f;
+        }
     }
+    if (ii) take(pi, 1);
   }
   // state scale: a power of two putting the largest start entry at most SMAX (columns keep
   // their norms under the unitary factors, so no later entry grows past it)
@@ -583,21 +643,29 @@ __global__ __launch_bounds__(NTH) void cm_cols_kernel(
   // ---- final raw state (z == 0): row-major planes through LDS column tiles
   if (z == 0) {
     float* tile = &sm.wpart[0][0][0];
+    const bool vec = planes_vec(h, fr, fi);
     for (int p = 0; p < 2; ++p) {
       if (part == p) {
 #pragma unroll
         for (int rt = 0; rt < TPW; ++rt)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = r0w + 32 * rt + 8 * (r >> 2) + 4 * g + (r & 3);
-            tile[ncol * HP + row] = hs[rt][r] * inv_ssc;
-          }
+          for (int r = 0; r < 16; ++r)
+            tile[(r0w + 32 * rt + 8 * (r >> 2) + 4 * g + (r & 3)) * TILE_LD + ncol] = hs[rt][r] * inv_ssc;
       }
       __syncthreads();
-      float* dst = p == 0 ? fr : fi;
-      for (int e = tid; e < h * COLS; e += NTH) {
-        const int r = e / COLS, cc = e % COLS;
-        if (c0 + cc < h) dst[b * hh + static_cast<int64_t>(r) * h + c0 + cc] = tile[cc * HP + r];
+      float* dst = (p == 0 ? fr : fi) + b * hh;
+      for (int e = tid; e < h * COLS / 4; e += NTH) {
+        const int r = e / 4, cc = c0 + 4 * (e % 4);
+        const float4 x = *reinterpret_cast<const float4*>(tile + r * TILE_LD + 4 * (e % 4));
+        float* d = dst + static_cast<int64_t>(r) * h + cc;
+        if (vec) {
+          if (cc < h) *reinterpret_cast<float4*>(d) = x;
+        } else {
+          if (cc < h) d[0] = x.x;
+          if (cc + 1 < h) d[1] = x.y;
+          if (cc + 2 < h) d[2] = x.z;
+          if (cc + 3 < h) d[3] = x.w;
+        }
       }
       __syncthreads();
     }
@@ -937,7 +1005,7 @@ hipError_t launch_typed(const IO* k, const IO* v, const float* coef, const float
   E* tt = static_cast<E*>(ws);
   E* yop = tt + static_cast<int64_t>(B) * nc * TT_STRIDE;  // [B][nc][HP / 16][64][8] f16
   if (nc > 0) {
-    hipLaunchKernelGGL((cm_prep_kernel<IO>), dim3(nc, B), dim3(64), 0, stream, k, v, coef, tt, yop, T, h,
+    hipLaunchKernelGGL((cm_prep_kernel<IO>), dim3(nc, B), dim3(64 * PWV), 0, stream, k, v, coef, tt, yop, T, h,
                        NWV * 32 * TPW);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -958,10 +1026,10 @@ hipError_t launch_scan16(const IO* q, const IO* k, const IO* v, const float* coe
   E* tt = static_cast<E*>(ws);
   E* yop = tt + static_cast<int64_t>(B) * nc * TT_STRIDE;
   if (fused)
-    hipLaunchKernelGGL((cm_prep_kernel<IO, true>), dim3(nc, B), dim3(64), 0, stream, k, v, coef, tt,
+    hipLaunchKernelGGL((cm_prep_kernel<IO, true>), dim3(nc, B), dim3(64 * PWV), 0, stream, k, v, coef, tt,
                        yop, T, h, NWV * 32 * TPW, stride);
   else
-    hipLaunchKernelGGL((cm_prep_kernel<IO>), dim3(nc, B), dim3(64), 0, stream, k, v, coef, tt, yop,
+    hipLaunchKernelGGL((cm_prep_kernel<IO>), dim3(nc, B), dim3(64 * PWV), 0, stream, k, v, coef, tt, yop,
                        T, h, NWV * 32 * TPW, int64_t{0});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

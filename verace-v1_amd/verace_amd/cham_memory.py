@@ -27,7 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .hip_kernels import (cham_fused_scan_supported, cham_step_, cham_step_fused_,
-                          launch_cham_hip_update, launch_cham_hip_update_fused)
+                          launch_cham_hip_update, launch_cham_hip_update_fused, unit_rows)
 
 
 class ContinuousHolographicMemory(nn.Module):
@@ -72,9 +72,7 @@ class ContinuousHolographicMemory(nn.Module):
 
     def project(self, x: torch.Tensor, active_mask: Optional[torch.Tensor] = None):
         """q, k, v [B, T, h] and gamma [B, T] as the reference builds them (:128-155)."""
-        q = F.normalize(self.w_q(x), p=2, dim=-1)
-        k = F.normalize(self.w_k(x), p=2, dim=-1)
-        v = F.normalize(F.silu(self.w_v(x)), p=2, dim=-1)
+        q, k, v = unit_rows(self.w_q(x)), unit_rows(self.w_k(x)), unit_rows(F.silu(self.w_v(x)))
         gamma = 0.1 * torch.sigmoid(self.w_gamma(x))
         if active_mask is not None:
             am = active_mask
