@@ -377,6 +377,12 @@ int vmi_unit_rows(const void* x, int x_dtype, void* y, int y_dtype, int64_t rows
 int vmi_unit_rows_bwd(const void* x, int x_dtype, const void* dy, int y_dtype, void* dx, int64_t rows,
                       int64_t D, float eps, void* stream);
 
+/* y = x w^T for a few rows (the nn.Linear calls of a decode step at a small batch): x [M, K] with row
+ * stride x_stride, w [N, K], y [M, N], all of io_dtype, sums fp32.  M <= 16, x, w and x's rows 16-byte
+ * aligned, K a multiple of 16 bytes, otherwise VMI_ERR_UNSUPPORTED. */
+int vmi_rows_linear(const void* x, int64_t x_stride, const void* w, int io_dtype, void* y, int64_t M,
+                    int64_t N, int64_t K, void* stream);
+
 /* The element-wise steps between a layer's matrix products.  dtype is the type of every tensor
  * argument without a type of its own; rows are contiguous and 16-byte aligned, of whole 16-byte
  * pieces (otherwise VMI_ERR_UNSUPPORTED: run the tensor operations instead).  Sums are fp32.

@@ -53,6 +53,7 @@ EXPORTED = (
     "vmi_cham_ns_retraction",
     "vmi_unit_rows",
     "vmi_unit_rows_bwd",
+    "vmi_rows_linear",
     "vmi_situ_glu",
     "vmi_mcmoe_coef",
     "vmi_norm_add",
@@ -141,6 +142,8 @@ def _declare(lib):
     lib.vmi_cham_ns_retraction.argtypes = [vp, vp, vp, vp, i64, i64, i32, vp, sz, vp]
     lib.vmi_cham_ns_retraction.restype = i32
     f32 = ctypes.c_float
+    lib.vmi_rows_linear.argtypes = [vp, i64, vp, i32, vp, i64, i64, i64, vp]
+    lib.vmi_rows_linear.restype = i32
     lib.vmi_unit_rows.argtypes = [vp, i32, vp, i32, i64, i64, f32, vp]
     lib.vmi_unit_rows.restype = i32
     lib.vmi_unit_rows_bwd.argtypes = [vp, i32, vp, i32, vp, i64, i64, f32, vp]

@@ -28,6 +28,7 @@ import torch.nn.functional as F
 
 from .hip_kernels import (cham_fused_scan_supported, cham_step_, cham_step_fused_,
                           launch_cham_hip_update, launch_cham_hip_update_fused, unit_rows)
+from .layer_ops import rows_call, rows_linear
 
 
 class ContinuousHolographicMemory(nn.Module):
@@ -118,9 +119,9 @@ class ContinuousHolographicMemory(nn.Module):
     def step_before_norm_(self, x, hologram, readout=None, active_mask=None):
         """:meth:`step_` without its last step, the RMSNorm."""
         if self._fused_step(x):  # one projection GEMM; normalisation and gamma in the kernel
-            rec = cham_step_fused_(F.linear(x, self._stacked_weight()), self.holographic_dim,
+            rec = cham_step_fused_(rows_linear(x, self._stacked_weight()), self.holographic_dim,
                                    hologram, readout, active_mask)
         else:
             q, k, v, gamma = self.project(x, active_mask)
             rec = cham_step_(q, k, v, gamma, hologram, readout)
-        return self.w_out(rec.to(self.w_out.weight.dtype))
+        return rows_call(self.w_out, rec.to(self.w_out.weight.dtype))

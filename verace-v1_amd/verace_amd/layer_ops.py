@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
@@ -52,6 +53,39 @@ def _rows(*ts) -> bool:
 def _row_fits(d: int, dtype: torch.dtype) -> bool:
     n = 16 // dtype.itemsize
     return d % n == 0 and d <= 1024 * n
+
+
+def _few_rows(x: torch.Tensor, n: int, k: int) -> bool:
+    """Whether ``csrc/rows_linear.hip`` takes x [M, k] times [n, k]: M <= 16, x up to 32 KB, a row up
+    to 4 KB, the weight up to 16 MB.  The library spends 19.5 us of host time on such a product, the
+    kernel's call 11; on the device, in us, kernel / library: bf16 n3328 k1024 M1 2.9 / 4.5, M16
+    3.7 / 4.6; fp32 there M1 4.4 / 5.4, M16 5.6 / 5.6; bf16 n1536 k2048 M4 4.3 / 5.1,
+    M16 5.3 / 5.1; past the lines bf16 n6400 k2048 M1 6.5 / 5.9, n16384 k4096 M16 30 / 22."""
+    size = x.dtype.itemsize
+    return (0 < x.numel() <= 16 * k and x.numel() * size <= 32768 and k * size <= 4096 and 0 < n
+            and n * k * size <= 2 ** 24 and k * size % 16 == 0)
+
+
+def rows_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``F.linear(x, weight)`` of a decode step, x [B, 1, hidden]: a few rows on
+    ``csrc/rows_linear.hip``, more on the library."""
+    n, k = weight.shape
+    if (x.shape[-1] == k and _few_rows(x, n, k) and fusable(x)
+            and type(weight) in (torch.Tensor, nn.Parameter) and weight.dtype == x.dtype
+            and weight.device == x.device and _rows(x, weight)):
+        out = torch.empty((*x.shape[:-1], n), device=x.device, dtype=x.dtype)
+        _lib.check(_lib.load().vmi_rows_linear(_ptr(x), k, _ptr(weight), _lib.dtype_code(x.dtype), _ptr(out),
+                                               x.numel() // k, n, k, _lib.stream_handle(x.device)),
+                   "vmi_rows_linear")
+        return out
+    return F.linear(x, weight)
+
+
+def rows_call(linear, x: torch.Tensor) -> torch.Tensor:
+    """``linear(x)`` for a projection without bias, as :func:`rows_linear` where that is the same."""
+    if plain(linear, nn.Linear) and linear.bias is None:
+        return rows_linear(x, linear.weight)
+    return linear(x)
 
 
 def _norm_ok(norm, d: int, dtype: torch.dtype) -> bool:

@@ -31,6 +31,7 @@ from . import ops as _ops  # noqa: F401  (registers torch.ops.verace.*)
 from .hip_kernels import (fused_scan_supported, fused_step_supported, launch_sssd_hip_scan,
                           launch_sssd_hip_scan_fused, sssd_scan, sssd_step_, sssd_step_fused_,
                           unit_rows)
+from .layer_ops import rows_call, rows_linear
 
 
 def _traced(x: torch.Tensor) -> bool:
@@ -196,14 +197,14 @@ class SSSDAttention(nn.Module):
             if not rms_grad:
                 w = self.head_rmsnorm.weight
                 w = torch.ones(D, device=x.device) if w is None else w.detach()
-            o = sssd_step_fused_(F.linear(x, self._stacked_weight()), H, D, state, active_mask, w,
+            o = sssd_step_fused_(rows_linear(x, self._stacked_weight()), H, D, state, active_mask, w,
                                  self.head_rmsnorm.eps)
             if rms_grad:
                 o = self.head_rmsnorm(o)
         else:
             q, k, v, delta = self.project(x, active_mask)
             o = self.head_rmsnorm(sssd_step_(q, k, v, delta, state))
-        return self.w_out(o.reshape(b, 1, H * D))
+        return rows_call(self.w_out, o.reshape(b, 1, H * D))
 
     def _fused_step(self, x: torch.Tensor) -> bool:
         return (self.fuse_projections and x.shape[1] == 1
