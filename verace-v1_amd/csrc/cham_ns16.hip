@@ -26,11 +26,16 @@
 // the update H D reads F(H) and F(D^T).  The update's epilogue writes F(H') (next update) and
 // F(H'^T) (next Gram), the Gram's F(D^T); the last update also writes fp32 H'.
 //
-// Workgroup: 4 waves, 128 x 128 output tile (wave (wr, wc) owns the 64 x 64 quarter: 2 x 2
-// blocks of 32 x 32, real and imaginary accumulators = 128 fp32 per lane).  K runs in steps
-// of 16 through a 4-stage ring of 32 KB LDS stages filled by LDS-direct loads
-// (global_load_lds_dwordx4, one per 1 KB fragment, 8 per wave per step); one LDS barrier per
-// step.  Per step a wave issues 48 MFMAs (4 blocks x 4 real products x 3 split terms).
+// Workgroup: a square tile of 128 x 128 (8 waves) or 64 x 64 (4 waves); a wave owns a row pair of
+// 32 x 32 blocks, or one block, real and imaginary.  K runs in steps of 16 through a ring of LDS
+// stages (4 of 32 KB, 3 of 16 KB) filled by LDS-direct loads (global_load_lds_dwordx4, one per
+// 1 KB fragment, 4 per wave per step), one barrier per step; a step's fragments go to registers
+// while the step before multiplies.  What bounds it: the matrix cores take 384 clocks per narrow
+// step and CU, the LDS as many; a wide step is 1536 clocks of products and about 500 of barrier
+// and load issue.  The wide tile moves half the LDS bytes per product, but one of them fills a CU
+// and [1, 1024, 1024] has 36 and 64 of them: three narrow workgroups share a CU and cover each
+// other's barriers.  Three steps, with 128 x 128 tiles on 4 waves alone before:
+// [1, 1024]^2 455 -> 172 us, [4, 1024]^2 504 -> 485, [4, 512]^2 264 -> 112, [8, 128]^2 96 -> 41.
 #include "vmi_common.h"
 #include "vmi_dispatch.h"
 #include "vmi_mfma.h"
@@ -43,16 +48,27 @@ typedef mfma_t<E> MM;
 typedef MM::v8 V8;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int TM = 128;            // output tile side
-constexpr int NT = 256;            // 4 waves
+constexpr int TM = 128;            // n is a multiple of it
+constexpr int NT = 256;            // the split kernel's 4 waves
 constexpr int FRAG = 512;          // f16 per fragment (64 lanes x 8)
-constexpr int NSTAGE = 4;
-constexpr int STAGE_FRAGS = 32;    // A and B: 4 blocks x (re, im) x (hi, lo)
 constexpr float SC = 256.f;        // operand scale
 constexpr float INV_SC2 = 1.f / (SC * SC);
-constexpr int EP_LD = TM + 4;      // epilogue tile pitch (floats)
-constexpr size_t SMEM = static_cast<size_t>(NSTAGE) * STAGE_FRAGS * FRAG * sizeof(E);  // 128 KB
-static_assert(SMEM >= static_cast<size_t>(TM) * EP_LD * sizeof(float), "epilogue tile fits");
+
+// A tile of NB x NB blocks of 32 x 32, its 2 x NB waves owning NB / 2 x 1 blocks each.
+template <int NB>
+struct Tile {
+  static constexpr int SIDE = 32 * NB;
+  static constexpr int THREADS = 128 * NB;
+  static constexpr int XB = NB / 2;             // block rows of a wave
+  static constexpr int STAGE_FRAGS = 8 * NB;    // A and B: NB blocks x (re, im) x (hi, lo)
+  static constexpr int LOADS = 4;               // LDS-direct loads per wave and step
+  static constexpr int NSTAGE = NB == 4 ? 4 : 3;
+  static constexpr int PER_SIMD = NB == 4 ? 2 : 3;  // waves: one workgroup on a CU, or three
+  static constexpr int EP_LD = SIDE + 4;        // epilogue tile pitch (floats)
+  static constexpr size_t SMEM = static_cast<size_t>(NSTAGE) * STAGE_FRAGS * FRAG * sizeof(E);
+  static_assert(SMEM >= static_cast<size_t>(SIDE) * EP_LD * sizeof(float), "epilogue tile fits");
+  static_assert(SMEM * (NB == 4 ? 1 : 3) <= 160 * 1024, "LDS of a CU");
+};
 
 // f16 offset of fragment (mb, kb), half hl, in an F array with nkb = n / 16 k-blocks
 __device__ __forceinline__ int64_t frag_off(int mb, int kb, int hl, int nkb) {
@@ -141,12 +157,22 @@ __device__ __forceinline__ V8 negate(V8 x) {
   return __builtin_bit_cast(V8, __builtin_bit_cast(u32x4, x) ^ 0x80008000u);
 }
 
-template <bool GRAM, bool LAST>
-__global__ __launch_bounds__(NT) void ns16_gemm_kernel(Args a) {
-  __shared__ __align__(16) unsigned char smem[SMEM];
+// One step's operand fragments of a wave: [block][re, im][hi, lo]
+template <int XB>
+struct Frags {
+  V8 a[XB][2][2];
+  V8 b[2][2];
+};
+
+template <bool GRAM, bool LAST, int NB>
+__global__ __launch_bounds__(Tile<NB>::THREADS, Tile<NB>::PER_SIMD) void ns16_gemm_kernel(Args a) {
+  typedef Tile<NB> TL;
+  constexpr int XB = TL::XB, NSTAGE = TL::NSTAGE, STAGE_FRAGS = TL::STAGE_FRAGS;
+  constexpr int EP_LD = TL::EP_LD, SIDE = TL::SIDE, BOFF = STAGE_FRAGS / 2;
+  __shared__ __align__(16) unsigned char smem[TL::SMEM];
   E* st = reinterpret_cast<E*>(smem);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wr = wave >> 1, wc = wave & 1;
+  const int wr = wave / NB, wc = wave % NB;
   const int n = a.n, nkb = n / 16, T = a.tiles_side;
 
   // XCD-aware order: workgroups dispatched to one XCD (g mod 8) take consecutive tiles, so
@@ -167,88 +193,94 @@ __global__ __launch_bounds__(NT) void ns16_gemm_kernel(Args a) {
   const int64_t nn = static_cast<int64_t>(n) * n;
   const int64_t moff = static_cast<int64_t>(mat) * 2 * nn;
 
-  // stage layout (fragments): [A: blk 4][re/im][hi/lo], then [B: blk 4][re/im][hi/lo]
-  const E* asrc[2] = {a.ar + moff, a.ai + moff};
-  const E* bsrc[2] = {a.br + moff, a.bi + moff};
+  // stage layout (fragments): [A: blk NB][re/im][hi/lo], then [B: blk NB][re/im][hi/lo]; a wave
+  // loads one part (re or im) of one block of A and of B.  A fragment pair (hi, lo) lies in 2 KB,
+  // the next step's right behind it in the F array.
+  const int blk = wave >> 1, im = wave & 1;
+  const E* ga = (im ? a.ai : a.ar) + moff + frag_off(NB * bi + blk, 0, 0, nkb) + lane * 8;
+  const E* gb = (im ? a.bi : a.br) + moff + frag_off(NB * bj + blk, 0, 0, nkb) + lane * 8;
+  const unsigned lds0 = lds_addr(smem) + wave * 2 * FRAG * sizeof(E);
   auto issue = [&](int ks, int s) {
-    E* sb = st + s * STAGE_FRAGS * FRAG;
+    const int64_t go = static_cast<int64_t>(ks) * 2 * FRAG;
+    const unsigned so = lds0 + s * STAGE_FRAGS * FRAG * sizeof(E);
+#pragma unroll
+    for (int hl = 0; hl < 2; ++hl) {
+      dma16(ga + go + hl * FRAG, so + hl * FRAG * sizeof(E));
+      dma16(gb + go + hl * FRAG, so + (BOFF + hl) * FRAG * sizeof(E));
+    }
+  };
+
+  f32x16 P[XB], Q[XB];
+#pragma unroll
+  for (int x = 0; x < XB; ++x) {
+    P[x] = f32x16{};
+    Q[x] = f32x16{};
+  }
+
+  const int nk = nkb;  // a multiple of 8
+#pragma unroll
+  for (int s = 0; s < NSTAGE - 1; ++s)
+    if (s < nk) issue(s, s);
+  // Fragments of step ks into registers: its loads landed, every wave is past step ks - 1's
+  // reads, whose stage takes the loads of step ks + NSTAGE - 1.
+  int slot = 0;  // ks % NSTAGE
+  auto read = [&](int ks, Frags<XB>& f) {
+    // this wave's loads of step ks are done once at most those of the NSTAGE - 2 steps issued
+    // after it remain
+    const int ahead = nk - 1 - ks;
+    if (ahead >= NSTAGE - 2) NS16_VMCNT((NSTAGE - 2) * TL::LOADS);
+    else if (NSTAGE > 3 && ahead == 1) NS16_VMCNT(TL::LOADS);
+    else NS16_VMCNT(0);
+    lds_barrier();
+    const E* sb = st + slot * STAGE_FRAGS * FRAG;
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int hl = 0; hl < 2; ++hl) {
-        dma16(asrc[p] + frag_off(4 * bi + wave, ks, hl, nkb) + lane * 8,
-              lds_addr(sb + ((wave * 2 + p) * 2 + hl) * FRAG));
-        dma16(bsrc[p] + frag_off(4 * bj + wave, ks, hl, nkb) + lane * 8,
-              lds_addr(sb + (16 + (wave * 2 + p) * 2 + hl) * FRAG));
+#pragma unroll
+        for (int x = 0; x < XB; ++x)
+          f.a[x][p][hl] = lds_frag(sb + (((XB * wr + x) * 2 + p) * 2 + hl) * FRAG, lane);
+        f.b[p][hl] = lds_frag(sb + (BOFF + (wc * 2 + p) * 2 + hl) * FRAG, lane);
       }
+    if (ks + NSTAGE - 1 < nk) issue(ks + NSTAGE - 1, slot == 0 ? NSTAGE - 1 : slot - 1);
+    slot = slot == NSTAGE - 1 ? 0 : slot + 1;
   };
-
-  f32x16 P[2][2], Q[2][2];
+  // GRAM: P += Ar Br + Ai Bi, Q += Ar Bi - Ai Br;  update: P += Ar Br - Ai Bi, Q += Ar Bi + Ai Br
+  auto multiply = [&](const Frags<XB>& f) {
+    V8 neg[XB][2];
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < XB; ++x)
 #pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      P[x][y] = f32x16{};
-      Q[x][y] = f32x16{};
-    }
-
-  const int nk = nkb;
-#pragma unroll
-  for (int s = 0; s < NSTAGE - 1; ++s)
-    if (s < nk) issue(s, s);
-  for (int ks = 0; ks < nk; ++ks) {
-    // this wave's loads of step ks are done once at most those of the next two steps remain
-    const int ahead = nk - 1 - ks;
-    if (ahead >= 2) NS16_VMCNT(16);
-    else if (ahead == 1) NS16_VMCNT(8);
-    else NS16_VMCNT(0);
-    lds_barrier();  // every wave's step-ks loads landed; every wave is done with step ks-1
-    if (ks + NSTAGE - 1 < nk) issue(ks + NSTAGE - 1, (ks + NSTAGE - 1) % NSTAGE);
-    const E* sb = st + (ks % NSTAGE) * STAGE_FRAGS * FRAG;
-    V8 arh[2], arl[2], aih[2], ail[2], brh[2], brl[2], bih[2], bil[2];
-#pragma unroll
-    for (int x = 0; x < 2; ++x) {
-      const int blk = 2 * wr + x;
-      arh[x] = lds_frag(sb + ((blk * 2 + 0) * 2 + 0) * FRAG, lane);
-      arl[x] = lds_frag(sb + ((blk * 2 + 0) * 2 + 1) * FRAG, lane);
-      aih[x] = lds_frag(sb + ((blk * 2 + 1) * 2 + 0) * FRAG, lane);
-      ail[x] = lds_frag(sb + ((blk * 2 + 1) * 2 + 1) * FRAG, lane);
-    }
-#pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      const int blk = 2 * wc + y;
-      brh[y] = lds_frag(sb + (16 + (blk * 2 + 0) * 2 + 0) * FRAG, lane);
-      brl[y] = lds_frag(sb + (16 + (blk * 2 + 0) * 2 + 1) * FRAG, lane);
-      bih[y] = lds_frag(sb + (16 + (blk * 2 + 1) * 2 + 0) * FRAG, lane);
-      bil[y] = lds_frag(sb + (16 + (blk * 2 + 1) * 2 + 1) * FRAG, lane);
-    }
-    // GRAM: P += Ar Br + Ai Bi, Q += Ar Bi - Ai Br;  update: P += Ar Br - Ai Bi, Q += Ar Bi + Ai Br
-    V8 nih[2], nil[2];
-#pragma unroll
-    for (int x = 0; x < 2; ++x) {
-      nih[x] = negate(aih[x]);
-      nil[x] = negate(ail[x]);
-    }
-#define NS16_TERM(ACC, XH, XL, YH, YL)                                 \
-  _Pragma("unroll") for (int x = 0; x < 2; ++x)                         \
-  _Pragma("unroll") for (int y = 0; y < 2; ++y)                         \
-    ACC[x][y] = MM::mma32(XH[x], YH[y], ACC[x][y]);                     \
-  _Pragma("unroll") for (int x = 0; x < 2; ++x)                         \
-  _Pragma("unroll") for (int y = 0; y < 2; ++y)                         \
-    ACC[x][y] = MM::mma32(XH[x], YL[y], ACC[x][y]);                     \
-  _Pragma("unroll") for (int x = 0; x < 2; ++x)                         \
-  _Pragma("unroll") for (int y = 0; y < 2; ++y)                         \
-    ACC[x][y] = MM::mma32(XL[x], YH[y], ACC[x][y]);
-    NS16_TERM(P, arh, arl, brh, brl)
-    NS16_TERM(Q, arh, arl, bih, bil)
+      for (int hl = 0; hl < 2; ++hl) neg[x][hl] = negate(f.a[x][1][hl]);
+    // hi*hi, hi*lo, lo*hi
+#define NS16_TERM(ACC, A, YP)                                                        \
+  _Pragma("unroll") for (int t = 0; t < 3; ++t)                                       \
+  _Pragma("unroll") for (int x = 0; x < XB; ++x)                                      \
+    ACC[x] = MM::mma32(A(x, t == 2), f.b[YP][t == 1], ACC[x]);
+#define NS16_RE(x, hl) f.a[x][0][hl]
+#define NS16_IM(x, hl) f.a[x][1][hl]
+#define NS16_NEG(x, hl) neg[x][hl]
+    NS16_TERM(P, NS16_RE, 0)
+    NS16_TERM(Q, NS16_RE, 1)
     if constexpr (GRAM) {
-      NS16_TERM(P, aih, ail, bih, bil)
-      NS16_TERM(Q, nih, nil, brh, brl)
+      NS16_TERM(P, NS16_IM, 1)
+      NS16_TERM(Q, NS16_NEG, 0)
     } else {
-      NS16_TERM(P, nih, nil, bih, bil)
-      NS16_TERM(Q, aih, ail, brh, brl)
+      NS16_TERM(P, NS16_NEG, 1)
+      NS16_TERM(Q, NS16_IM, 0)
     }
 #undef NS16_TERM
+#undef NS16_RE
+#undef NS16_IM
+#undef NS16_NEG
+  };
+  Frags<XB> f0, f1;
+  read(0, f0);
+  for (int ks = 0; ks < nk; ks += 2) {  // the next step's fragments arrive during the products
+    read(ks + 1, f1);
+    multiply(f0);
+    if (ks + 2 < nk) read(ks + 2, f0);
+    multiply(f1);
   }
 
   // ---- epilogue: each output tile through LDS (pitch EP_LD floats), then F-layout writes
@@ -258,65 +290,93 @@ __global__ __launch_bounds__(NT) void ns16_gemm_kernel(Args a) {
 #pragma unroll
   for (int part = 0; part < 2; ++part) {
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < XB; ++x) {
+      const f32x16& acc = part == 0 ? P[x] : Q[x];
 #pragma unroll
-      for (int y = 0; y < 2; ++y) {
-        const f32x16& acc = part == 0 ? P[x][y] : Q[x][y];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = 64 * wr + 32 * x + 8 * (r >> 2) + 4 * g2 + (r & 3);
-          const int col = 64 * wc + 32 * y + l32;
-          float val;
-          if constexpr (GRAM) {  // Dr = 3I - P, Di = -Q
-            val = -acc[r] * INV_SC2;
-            if (part == 0 && bi == bj && row == col) val += 3.f;
-          } else {
-            val = 0.5f * INV_SC2 * acc[r];
-          }
-          ep[row * EP_LD + col] = val;
+      for (int r = 0; r < 16; ++r) {
+        const int row = 32 * (XB * wr + x) + 8 * (r >> 2) + 4 * g2 + (r & 3);
+        const int col = 32 * wc + l32;
+        float val;
+        if constexpr (GRAM) {  // Dr = 3I - P, Di = -Q
+          val = -acc[r] * INV_SC2;
+          if (part == 0 && bi == bj && row == col) val += 3.f;
+        } else {
+          val = 0.5f * INV_SC2 * acc[r];
         }
+        ep[row * EP_LD + col] = val;
       }
+    }
     lds_barrier();
     E* o1 = (part == 0 ? a.o1r : a.o1i) + moff;
-    // transposed write: F(C^T) blocks (mb over the tile's columns, kb over its rows); wave w
-    // takes column block w.  GRAM: into F(D^T) at (4 bj + w, 8 bi + kbl); update: F(H'^T).
+    // transposed write: F(C^T) blocks (mb over the tile's columns, kb over its rows); two waves
+    // share column block mb, half of its kb each.  GRAM: into F(D^T) at
+    // (NB bj + mb, 2 NB bi + kbl); update: F(H'^T).
+    const int mb = wave >> 1, kb0 = NB * (wave & 1);
     {
       E* dstT = GRAM ? o1 : (part == 0 ? a.o2r : a.o2i) + moff;
 #pragma unroll 2
-      for (int kbl = 0; kbl < 8; ++kbl) {
+      for (int kbl = kb0; kbl < kb0 + NB; ++kbl) {
         float xv[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xv[j] = ep[(16 * kbl + 8 * g2 + j) * EP_LD + 32 * wave + l32];
-        split_store(xv, 1.f, dstT + frag_off(4 * bj + wave, 8 * bi + kbl, 0, nkb), lane);
+        for (int j = 0; j < 8; ++j) xv[j] = ep[(16 * kbl + 8 * g2 + j) * EP_LD + 32 * mb + l32];
+        split_store(xv, 1.f, dstT + frag_off(NB * bj + mb, 2 * NB * bi + kbl, 0, nkb), lane);
       }
     }
-    // direct write: F(C) blocks (mb over rows, kb over columns); wave w takes row block w.
+    // direct write: F(C) blocks (mb over rows, kb over columns), waves as above.
     // GRAM: the mirror tile of F(D^T) (Dr symmetric: +, Di antisymmetric: -), off the diagonal
     // only; update: F(H').
     if (!GRAM || bi < bj) {
       const float sign = (GRAM && part == 1) ? -1.f : 1.f;
 #pragma unroll 2
-      for (int kbl = 0; kbl < 8; ++kbl) {
-        const float* src = ep + (32 * wave + l32) * EP_LD + 16 * kbl + 8 * g2;
+      for (int kbl = kb0; kbl < kb0 + NB; ++kbl) {
+        const float* src = ep + (32 * mb + l32) * EP_LD + 16 * kbl + 8 * g2;
         float xv[8];
         const float4 p0 = *reinterpret_cast<const float4*>(src);
         const float4 p1 = *reinterpret_cast<const float4*>(src + 4);
         xv[0] = p0.x; xv[1] = p0.y; xv[2] = p0.z; xv[3] = p0.w;
         xv[4] = p1.x; xv[5] = p1.y; xv[6] = p1.z; xv[7] = p1.w;
-        split_store(xv, sign, o1 + frag_off(4 * bi + wave, 8 * bj + kbl, 0, nkb), lane);
+        split_store(xv, sign, o1 + frag_off(NB * bi + mb, 2 * NB * bj + kbl, 0, nkb), lane);
       }
     }
     if constexpr (LAST) {  // fp32 H' rows
       float* f = (part == 0 ? a.fr : a.fi) + static_cast<int64_t>(mat) * nn;
 #pragma unroll 4
-      for (int i = tid; i < TM * TM / 4; i += NT) {
-        const int row = i / (TM / 4), c4 = i - row * (TM / 4);
-        *reinterpret_cast<float4*>(f + static_cast<int64_t>(TM * bi + row) * n + TM * bj + 4 * c4) =
+      for (int i = tid; i < SIDE * SIDE / 4; i += TL::THREADS) {
+        const int row = i / (SIDE / 4), c4 = i - row * (SIDE / 4);
+        *reinterpret_cast<float4*>(f + static_cast<int64_t>(SIDE * bi + row) * n + SIDE * bj + 4 * c4) =
             *reinterpret_cast<const float4*>(ep + row * EP_LD + 4 * c4);
       }
     }
     lds_barrier();  // before the next part overwrites the tile
   }
+}
+
+// Which tile: wide ones run in rounds of one per CU, each about 80 us at n 1024 however full it
+// is, narrow ones cost 24.5 us per 256 of them.  So wide only where their rounds are nearly full:
+// at least 850 narrow tiles per round (measured over batches 1 to 12 of n 1024 and n 128 to 4096,
+// three steps: batch 4, both products wide 484, both narrow 505 us; batch 8, 972 and 911 us;
+// batch 1, 399 and 172 us; [8, 128], 84 and 41 us).
+constexpr int64_t CUS = 256, NARROW_PER_ROUND = 850;
+
+template <bool GRAM, bool LAST, int NB>
+hipError_t gemm_tiles(Args a, hipStream_t stream) {
+  const int t = a.n / Tile<NB>::SIDE;
+  a.tiles_side = t;
+  a.ntiles = GRAM ? t * (t + 1) / 2 : t * t;
+  a.total = (a.ntiles * a.batch + 7) / 8 * 8;
+  hipLaunchKernelGGL((ns16_gemm_kernel<GRAM, LAST, NB>), dim3(a.total), dim3(Tile<NB>::THREADS),
+                     0, stream, a);
+  return hipGetLastError();
+}
+
+template <bool GRAM, bool LAST>
+hipError_t gemm(const Args& a, hipStream_t stream) {
+  const int64_t t4 = a.n / Tile<4>::SIDE, t2 = a.n / Tile<2>::SIDE;
+  const int64_t wide = (GRAM ? t4 * (t4 + 1) / 2 : t4 * t4) * a.batch;
+  const int64_t narrow = (GRAM ? t2 * (t2 + 1) / 2 : t2 * t2) * a.batch;
+  return narrow >= NARROW_PER_ROUND * ((wide + CUS - 1) / CUS)
+             ? gemm_tiles<GRAM, LAST, 4>(a, stream)
+             : gemm_tiles<GRAM, LAST, 2>(a, stream);
 }
 
 }  // namespace ns16
@@ -341,36 +401,24 @@ hipError_t launch_ns16_retraction(const float* h_real, const float* h_imag, floa
   hipLaunchKernelGGL(ns16_split_kernel, dim3((nfr + 3) / 4, batch, 4), dim3(NT), 0, stream,
                      h_real, h_imag, hd[0][0], hd[0][1], ht[0], ht[1], n);
   hipError_t e = hipGetLastError();
-  const int T = n / TM;
   for (int s = 0; s < steps && e == hipSuccess; ++s) {
     const int cur = s & 1, nxt = cur ^ 1;
     Args g{};
     g.n = n;
     g.batch = batch;
-    g.tiles_side = T;
     // Gram: A = B = F(H^T)
     g.ar = ht[0]; g.ai = ht[1]; g.br = ht[0]; g.bi = ht[1];
     g.o1r = dt[0]; g.o1i = dt[1];
-    g.ntiles = T * (T + 1) / 2;
-    g.total = (g.ntiles * batch + 7) / 8 * 8;
-    hipLaunchKernelGGL((ns16_gemm_kernel<true, false>), dim3(g.total), dim3(NT), 0, stream, g);
-    e = hipGetLastError();
+    e = gemm<true, false>(g, stream);
     if (e != hipSuccess) break;
     // update: A = F(H), B = F(D^T); writes F(H') into the other buffer and F(H'^T) over F(H^T)
     Args u{};
     u.n = n;
     u.batch = batch;
-    u.tiles_side = T;
     u.ar = hd[cur][0]; u.ai = hd[cur][1]; u.br = dt[0]; u.bi = dt[1];
     u.o1r = hd[nxt][0]; u.o1i = hd[nxt][1]; u.o2r = ht[0]; u.o2i = ht[1];
     u.fr = out_real; u.fi = out_imag;
-    u.ntiles = T * T;
-    u.total = (u.ntiles * batch + 7) / 8 * 8;
-    if (s + 1 == steps)
-      hipLaunchKernelGGL((ns16_gemm_kernel<false, true>), dim3(u.total), dim3(NT), 0, stream, u);
-    else
-      hipLaunchKernelGGL((ns16_gemm_kernel<false, false>), dim3(u.total), dim3(NT), 0, stream, u);
-    e = hipGetLastError();
+    e = s + 1 == steps ? gemm<false, true>(u, stream) : gemm<false, false>(u, stream);
   }
   return e;
 }
