@@ -24,7 +24,8 @@
 // (2 KB per fragment pair), so every fragment load is one contiguous 1 KB.  The B operand of
 // X Y is the A-operand fragment of Y^T, so the Gram H^T H reads F(H^T) for both operands and
 // the update H D reads F(H) and F(D^T).  The update's epilogue writes F(H') (next update) and
-// F(H'^T) (next Gram), the Gram's F(D^T); the last update also writes fp32 H'.
+// F(H'^T) (next Gram), the Gram's F(D^T); the last update writes
+// fp32 H' alone (79 us at [4, 1024]^2; with the fragments, which nothing read, 94).
 //
 // Workgroup: a square tile of 128 x 128 (8 waves) or 64 x 64 (4 waves); a wave owns a row pair of
 // 32 x 32 blocks, or one block, real and imaginary.  K runs in steps of 16 through a ring of LDS
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(Tile<NB>::THREADS, Tile<NB>::PER_SIMD) void ns16_ge
     // share column block mb, half of its kb each.  GRAM: into F(D^T) at
     // (NB bj + mb, 2 NB bi + kbl); update: F(H'^T).
     const int mb = wave >> 1, kb0 = NB * (wave & 1);
-    {
+    if constexpr (!LAST) {
       E* dstT = GRAM ? o1 : (part == 0 ? a.o2r : a.o2i) + moff;
 #pragma unroll 2
       for (int kbl = kb0; kbl < kb0 + NB; ++kbl) {
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(Tile<NB>::THREADS, Tile<NB>::PER_SIMD) void ns16_ge
     // direct write: F(C) blocks (mb over rows, kb over columns), waves as above.
     // GRAM: the mirror tile of F(D^T) (Dr symmetric: +, Di antisymmetric: -), off the diagonal
     // only; update: F(H').
-    if (!GRAM || bi < bj) {
+    if (!LAST && (!GRAM || bi < bj)) {
       const float sign = (GRAM && part == 1) ? -1.f : 1.f;
 #pragma unroll 2
       for (int kbl = kb0; kbl < kb0 + NB; ++kbl) {
