@@ -86,11 +86,12 @@ int vmi_sssd_scan_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D,
  * Arithmetic: F32 I/O, D != 128 and T < 32 run in fp32: in chunks of 16 tokens on the fp32
  * matrix cores for 5 <= T and D <= 128, given the workspace of vmi_sssd_scan_workspace_bytes
  * (optional for these calls: without it, or with less, they run token by token, as T < 5,
- * D > 128 and any sequence with a rotation m > 0.25 or a non-finite token always do).
- * BF16 / F16 I/O with
- * D = 128 and T >= 32 run the chunk-parallel scan, whose matrix-core operands (the state, W
- * and Z, once per 16-token chunk) are f16 with fp32 accumulation.  That holds the 2e-2
- * relative / 1e-4 norm-drift bars while every token's rotation
+ * D > 128 and any sequence with a non-finite token or one of ((delta / 2) |k| |v|)^2 > 0.003
+ * always do: past that bound the chunk form would round worse than the token-by-token one; unit
+ * k, v with delta <= 0.1 stay below 0.0026).
+ * BF16 / F16 I/O with D = 128 and T >= 32 run the chunk-parallel scan, whose matrix-core operands
+ * (the state, W and Z, once per 16-token chunk) are f16 with fp32 accumulation.  That holds the
+ * 2e-2 relative / 1e-4 norm-drift bars while every token's rotation
  * m = (delta/2) |k| |v| sin(angle(k, v)) stays <= 0.25 (measured to T = 65536); unit k, v
  * with delta <= 0.1 (the SSSD module's inputs) give m <= 0.05.  A
  * sequence with any token above m = 0.25 is detected on the device and recomputed in fp32

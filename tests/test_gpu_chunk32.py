@@ -6,6 +6,7 @@ Bars: fp32 I/O 1e-5 relative Frobenius error per (b, h) slice (the repository's 
 5e-8 .. 1.2e-6 here, the token-sequential scan 1e-7 .. 3.4e-6); 16-bit I/O: the output within one
 rounding of the type (2^-8 / 2^-11), the fp32 state at 1e-5."""
 import ctypes
+import math
 
 import numpy as np
 import pytest
@@ -102,25 +103,67 @@ def test_chunk32_unaligned_rows(device, dtype, D, offset):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
 
 
+def _pairs(T, D, length, angle, skew, distinct, seed):
+    """Tokens with |k| = |v| = length, the given angle between k and v and (delta / 2) |k| |v| = skew,
+    taken in turn from ``distinct`` k, v pairs (few repeated pairs are what the chunk's substitution
+    cancels worst on)."""
+    g = torch.Generator().manual_seed(seed)
+    k, w = (F.normalize(torch.randn(2, distinct, D, generator=g), dim=-1) for _ in range(2))
+    w = F.normalize(w - (w * k).sum(-1, keepdim=True) * k, dim=-1)
+    v = math.cos(angle) * k + math.sin(angle) * w
+    turn = torch.arange(T) % distinct
+    k, v = (length * t[:, turn].transpose(0, 1)[None] for t in (k, v))
+    q = F.normalize(torch.randn(1, T, 2, D, generator=g), dim=-1)
+    delta = torch.full((1, T, 2), 2.0 * skew / length ** 2)
+    return q, k.contiguous(), v.contiguous(), delta
+
+
 def test_chunk32_related_tokens(device):
     """Tokens whose k and v are nearly the same vectors all along (the Gram matrix of a chunk is
-    close to rank 2), rotating by the most that the chunk form takes (m <= 0.25)."""
+    close to rank 2), at the largest delta that the chunk form takes of unit k, v."""
     B, T, H, D = 1, 600, 2, 64
-    q, k, v, delta, psi0 = _inputs(B, T, H, D, torch.float32, 8, delta_scale=0.49)
+    q, k, v, delta, psi0 = _inputs(B, T, H, D, torch.float32, 8, delta_scale=0.109)
     k = F.normalize(k[:, :1] + 1e-2 * k, dim=-1)
     v = F.normalize(v[:, :1] + 1e-2 * v, dim=-1)
     o64, p64 = _oracle(q, k, v, delta, psi0)
     o, psi = _c_scan(q, k, v, delta, psi0, device)
     print(f"[case] chunk32 related tokens: o {_slice_err(o, o64, (1, 3)):.1e} psi {_slice_err(psi, p64, (2, 3)):.1e}", flush=True)
     assert _slice_err(o, o64, (1, 3)) <= 1e-5 and _slice_err(psi, p64, (2, 3)) <= 1e-5
+    assert not torch.equal(psi, _c_scan(q, k, v, delta, psi0, device, workspace=False)[1])
+
+
+@pytest.mark.parametrize("length", [1.0, 3.0, 10.0, 30.0])
+@pytest.mark.parametrize("angle", [1.5, 0.1, 0.01, 0.003])
+@pytest.mark.parametrize("skew", [0.054, 0.06, 0.5, 5.0])
+def test_chunk32_never_rounds_worse_than_the_sequential_scan(device, length, angle, skew):
+    """Nearly parallel k and v rotate little however long they are, but T~'s terms grow with
+    (delta / 2) |k| |v|: past its bound (0.0547) a call is the token-sequential scan's bits, below it
+    no more than twice as far from fp64 (1.5 measured over tokens of this kind), both sides' few last
+    bits (2e-7) apart."""
+    D, T = 64, 256
+    if skew * math.sin(angle) > 0.25:
+        skew = 0.25 / math.sin(angle)   # the rotation m stays where the 16-bit scan's rule has it
+    for distinct in (2, 3):
+        q, k, v, delta = _pairs(T, D, length, angle, skew, distinct, 7)
+        o, psi = _c_scan(q, k, v, delta, None, device)
+        os, ps = _c_scan(q, k, v, delta, None, device, workspace=False)
+        if skew > 0.055:
+            assert torch.equal(o, os) and torch.equal(psi, ps)
+            continue
+        assert not torch.equal(psi, ps)
+        o64, p64 = _oracle(q, k, v, delta, None)
+        for x, xs, ref, dims in ((o, os, o64, (1, 3)), (psi, ps, p64, (2, 3))):
+            e, es = _slice_err(x, ref, dims), _slice_err(xs, ref, dims)
+            print(f"[case] chunk32 length {length} angle {angle} skew {skew:.3f}: {e:.1e} ({es:.1e})", flush=True)
+            assert e <= 2.0 * es + 2e-7
 
 
 def test_chunk32_wide_and_nonfinite_sequences_take_the_sequential_scan(device):
-    """A sequence with a token above the chunk form's rotation limit, or one whose Cayley factor
+    """A sequence with a token above the chunk form's limit, or one whose Cayley factor
     is not finite, gives the token-sequential scan's bits; the others the chunk result."""
     B, T, H, D = 1, 700, 4, 64
     q, k, v, delta, psi0 = _inputs(B, T, H, D, torch.float32, 9)
-    delta[0, 500, 1] = 3.0           # m up to 1.5
+    delta[0, 500, 1] = 3.0           # (delta / 2) |k| |v| = 1.5
     k[0, 3, 2, 5] = float("nan")
     v[0, T - 1, 3, 0] = float("inf")
     o, psi = _c_scan(q, k, v, delta, psi0, device)

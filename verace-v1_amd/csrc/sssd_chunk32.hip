@@ -41,6 +41,7 @@ constexpr int R = 32;     // rank rows of a chunk
 constexpr int TTP = 36;   // T~ row pitch (floats): 16-byte rows, conflict-free 16-byte reads
 constexpr int LX = 20;    // X row pitch: the four 16-lane groups of a write in distinct banks
 constexpr int MAX_SEG = 64;
+constexpr float kMaxSkew2 = 0.003f;  // largest ((delta / 2) |k| |v|)^2 of a token (c32_prep_kernel)
 
 // Four consecutive elements of a row as they lie in memory.
 template <typename IO> struct Raw4 { uint2 w; };
@@ -170,7 +171,14 @@ __global__ __launch_bounds__(64 * PW) void c32_prep_kernel(
     bool ok;
     const cayley2 m = cayley_guarded(dl, kk, vv, kv, ok);
     Ms[wave][t] = make_float4(m.m00, m.m01, m.m10, m.m11);
-    out = !ok || rotation_outside_chunk_envelope(dl, kk, vv, kv);
+    // Rounding of T~.  Its terms have the size of s = (delta / 2) |k| |v| (the rotation's m is
+    // s sin(angle(k, v)), much smaller where k and v are nearly parallel) and cancel over the chunk's
+    // substitution.  In fp32 against fp64 (adversarial tokens: few distinct near-parallel pairs
+    // repeated), the state's error over the token-sequential scan's is at most 1.5 at s^2 <= 0.003,
+    // 2.3 at 0.005, 4 at 0.01, 20 at 0.06, and without a bound on s the state is lost (0.4 relative
+    // at |k| = |v| = 30, angle 0.003, m = 0.135).  Unit k, v and delta <= 0.1 give s^2 <= 0.0025.
+    const float s = 0.5f * dl;
+    out = !ok || (s * kk) * (s * vv) > kMaxSkew2;
   }
   const uint64_t any = __ballot(out);
   __builtin_amdgcn_wave_barrier();
@@ -298,6 +306,8 @@ __global__ __launch_bounds__(4 * DP) void c32_pass_kernel(Args a) {
   };
 
   if (c0 < c1) fetch(c0);
+  uint32_t flagged = 0;
+  for (int c = c0 + tid; c < c1; c += NT) flagged |= a.flags[static_cast<int64_t>(bh) * a.nch + c];
   // state: tile S, register r = row 16 S + 4 g + r of column 16 wave + l16
   f32x4 psi[SS];
   {
@@ -331,7 +341,12 @@ __global__ __launch_bounds__(4 * DP) void c32_pass_kernel(Args a) {
     }
   }
   if (c0 < c1) commit(0);
-  lds_barrier();
+  {  // Inputs visible.  With a flagged chunk the sequence runs again token by token, which writes all
+     // of it, so this segment ends here: a call whose sequences are all flagged pays the preparation.
+    const int any = __syncthreads_or(flagged != 0);
+    if (READOUT && tid == 0) a.seg_flags[static_cast<int64_t>(bh) * a.nseg + seg] = any != 0;
+    if (any) return;
+  }
   for (int c = c0; c < c1; ++c) {
     const int p = (c - c0) & 1;
     const float *U = UT[p], *Tt = TT[p], *Q = QT[p];
@@ -470,12 +485,6 @@ __global__ __launch_bounds__(4 * DP) void c32_pass_kernel(Args a) {
         }
       }
     }
-  }
-  if (READOUT) {  // does a chunk of this segment need the token-sequential scan?
-    uint32_t f = 0;
-    for (int c = c0 + tid; c < c1; c += NT) f |= a.flags[static_cast<int64_t>(bh) * a.nch + c];
-    const int any = __syncthreads_or(f != 0);
-    if (tid == 0) a.seg_flags[static_cast<int64_t>(bh) * a.nseg + seg] = any != 0;
   }
   // end state
   if (READOUT && seg != a.nseg - 1) return;
