@@ -1,0 +1,46 @@
+"""What the fused layer steps may take, checked on the host with fake device tensors: parameters that
+the torch ops refuse, convert or broadcast (another shape, type, device or tensor class) must reach those
+ops, as the kernels read them as they stand.  (No case here may run on a device: a kernel given a
+shorter weight would read past it.)"""
+import pytest
+import torch
+import torch.nn as nn
+from torch._subclasses.fake_tensor import FakeTensor, FakeTensorMode
+
+from verace_amd import layer_ops
+
+D = 64
+
+
+@pytest.fixture
+def mode(monkeypatch):
+    """Fake tensors on cuda devices count as plain, aligned device tensors."""
+    monkeypatch.setattr(layer_ops, "fusable", lambda x: True)
+    monkeypatch.setattr(layer_ops, "_rows", lambda *ts: all(t is None or t.is_contiguous() for t in ts))
+    monkeypatch.setattr(layer_ops, "_PLAIN", (torch.Tensor, nn.Parameter, FakeTensor), raising=False)
+    return FakeTensorMode(allow_non_fake_inputs=True)
+
+
+def _halting(mode, linear, threshold=0.9):
+    with mode:
+        h = torch.empty(2, 3, D, device="cuda:0")
+        acc = torch.empty(2, 3, device="cuda:0")
+    return layer_ops.HaltingState.start(linear(), threshold, h, h, acc, acc)
+
+
+@pytest.mark.parametrize("change", ["narrow", "wide", "two outputs", "device", "bias device", "bias shape",
+                                    "bias type", "no bias", "threshold"])
+def test_halting_unit_must_fit(mode, change):
+    def linear(change):
+        with mode:
+            d = {"narrow": D // 2, "wide": 2 * D}.get(change, D)
+            m = nn.Linear(d, 2 if change == "two outputs" else 1, bias=change != "no bias",
+                          device="cuda:1" if change == "device" else "cuda:0")
+            b = {"bias device": dict(device="cuda:1"), "bias shape": dict(device="cuda:0"),
+                 "bias type": dict(device="cuda:0", dtype=torch.float16)}.get(change)
+            if b is not None:
+                m.bias = nn.Parameter(torch.empty(2 if change == "bias shape" else 1, **b))
+        return m
+    assert _halting(mode, lambda: linear("")) is not None
+    threshold = torch.tensor(0.9) if change == "threshold" else 0.9
+    assert _halting(mode, lambda: linear(change), threshold) is None

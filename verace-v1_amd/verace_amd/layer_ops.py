@@ -50,6 +50,15 @@ def _rows(*ts) -> bool:
     return all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for t in ts)
 
 
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
+def _parameter_ok(p, shape: tuple, x: torch.Tensor) -> bool:
+    """A plain tensor of exactly ``shape`` beside ``x``, in its type: what torch's op would refuse or
+    convert must reach that op."""
+    return type(p) in _PLAIN and tuple(p.shape) == shape and p.dtype == x.dtype and p.device == x.device
+
+
 def _row_fits(d: int, dtype: torch.dtype) -> bool:
     n = 16 // dtype.itemsize
     return d % n == 0 and d <= 1024 * n
@@ -166,10 +175,10 @@ class HaltingState:
 
     @staticmethod
     def start(linear, threshold, h, final_h, acc, depth) -> Optional["HaltingState"]:
-        w, b = linear.weight, linear.bias
-        ok = (fusable(h) and plain(linear, nn.Linear) and b is not None and w.dtype == h.dtype
-              and b.dtype == h.dtype and w.is_cuda and h.numel() > 0 and _row_fits(h.shape[-1], h.dtype)
-              and _rows(h, final_h, w))
+        d = h.shape[-1]
+        ok = (fusable(h) and plain(linear, nn.Linear) and isinstance(threshold, (int, float))
+              and _parameter_ok(linear.weight, (1, d), h) and _parameter_ok(linear.bias, (1,), h)
+              and h.numel() > 0 and _row_fits(d, h.dtype) and _rows(h, final_h, linear.weight))
         return HaltingState(linear, threshold, final_h, acc, depth) if ok else None
 
     def _run(self, out, h, h_next, active, still, mode: int) -> None:
@@ -180,7 +189,8 @@ class HaltingState:
             _lib.stream_handle(h.device)), "vmi_halting_update")
 
     def accepts(self, out: torch.Tensor, h: torch.Tensor) -> bool:
-        return fusable(out) and out.dtype == h.dtype and out.shape == h.shape and _rows(out, h)
+        return (fusable(out) and out.dtype == h.dtype and out.device == h.device and out.shape == h.shape
+                and _rows(out, h))
 
     def step(self, out, h, active, below_min_depth: bool):
         """The next (h, active)."""
