@@ -9,6 +9,8 @@ from torch._subclasses.fake_tensor import FakeTensor, FakeTensorMode
 
 from verace_amd import layer_ops
 
+pytestmark = pytest.mark.filterwarnings("ignore:Accessing the data pointer of FakeTensor")
+
 D = 64
 
 
@@ -44,3 +46,36 @@ def test_halting_unit_must_fit(mode, change):
     assert _halting(mode, lambda: linear("")) is not None
     threshold = torch.tensor(0.9) if change == "threshold" else 0.9
     assert _halting(mode, lambda: linear(change), threshold) is None
+
+
+@pytest.mark.parametrize("change", ["shorter", "longer", "device", "type", "no weight", "other shape"])
+@pytest.mark.parametrize("place", ["norm1", "norm2"])
+def test_norm_weight_must_fit(mode, monkeypatch, change, place):
+    """norm_add with a replaced RMSNorm weight goes to the module's call (which refuses or converts)."""
+    taken = []
+    monkeypatch.setattr(layer_ops._lib, "load", lambda: taken.append("kernel") or _Lib())
+    monkeypatch.setattr(layer_ops._lib, "stream_handle", lambda device: None)
+    monkeypatch.setattr(nn.RMSNorm, "forward", lambda self, x: taken.append("module") or x)
+    with mode:
+        a = torch.empty(3, D, device="cuda:0")
+        norm = nn.RMSNorm(D, device="cuda:0")
+        layer_ops.norm_add(a, **{place: norm})
+        assert taken == ["kernel"]
+        if change == "no weight":
+            norm = nn.RMSNorm(D, elementwise_affine=False)
+        elif change == "other shape":
+            norm = nn.RMSNorm((3, D), device="cuda:0")
+        else:
+            norm.weight = nn.Parameter(torch.empty(
+                {"shorter": D // 2, "longer": 2 * D}.get(change, D),
+                device="cuda:1" if change == "device" else "cuda:0",
+                dtype=torch.float16 if change == "type" else torch.float32))
+        layer_ops.norm_add(a, **{place: norm})
+    assert taken == ["kernel", "module"]
+
+
+class _Lib:
+    """Every entry point of the library, doing nothing."""
+
+    def __getattr__(self, name):
+        return lambda *args: 0

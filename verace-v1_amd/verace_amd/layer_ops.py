@@ -97,10 +97,10 @@ def rows_call(linear, x: torch.Tensor) -> torch.Tensor:
     return linear(x)
 
 
-def _norm_ok(norm, d: int, dtype: torch.dtype) -> bool:
-    return norm is None or (plain(norm, nn.RMSNorm) and norm.weight is not None
-                            and tuple(norm.normalized_shape) == (d,) and norm.weight.dtype == dtype
-                            and norm.weight.is_cuda and _rows(norm.weight))
+def _norm_ok(norm, x: torch.Tensor) -> bool:
+    d = x.shape[-1]
+    return norm is None or (plain(norm, nn.RMSNorm) and tuple(norm.normalized_shape) == (d,)
+                            and _parameter_ok(norm.weight, (d,), x) and _rows(norm.weight))
 
 
 def _eps(norm, dtype) -> float:
@@ -116,7 +116,7 @@ def norm_add(a: torch.Tensor, norm1=None, c: Optional[torch.Tensor] = None,
     same = all(t is None or (type(t) is torch.Tensor and t.dtype == a.dtype and t.shape == a.shape
                              and t.device == a.device) for t in (b, c))
     if (fusable(a) and same and a.numel() > 0 and _row_fits(d, a.dtype) and _rows(a, b, c)
-            and _norm_ok(norm1, d, a.dtype) and _norm_ok(norm2, d, a.dtype)):
+            and _norm_ok(norm1, a) and _norm_ok(norm2, a)):
         s = torch.empty_like(a)
         out = None if norm2 is None else torch.empty_like(a)
         _lib.check(_lib.load().vmi_norm_add(
