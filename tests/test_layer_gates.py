@@ -74,6 +74,44 @@ def test_norm_weight_must_fit(mode, monkeypatch, change, place):
     assert taken == ["kernel", "module"]
 
 
+@pytest.mark.parametrize("change", ["router", "sigma", "sigma device", "sigma type", "vproj rows"])
+def test_mcmoe_coefficients_must_fit(mode, monkeypatch, change):
+    """Logits, sigma or projections of other sizes than the module's go to the torch ops."""
+    taken = []
+    monkeypatch.setattr(layer_ops._lib, "load", lambda: taken.append("kernel") or _Lib())
+    monkeypatch.setattr(layer_ops._lib, "stream_handle", lambda device: None)
+    n, C, r = 5, 16, 8
+
+    def make(rows, cols, **kw):
+        return torch.empty(rows, cols, **{"device": "cuda:0", **kw})
+    with mode:
+        good = make(n, C), make(n, C * r), make(n, C * r)
+        layer_ops.mcmoe_coef(*good, 4, C)
+        assert taken == ["kernel"]
+        bad = list(good)
+        i, t = {"router": (0, make(n, C // 2)), "sigma": (1, make(n, C * r // 2)),
+                "sigma device": (1, make(n, C * r, device="cuda:1")),
+                "sigma type": (1, make(n, C * r, dtype=torch.float16)),
+                "vproj rows": (2, make(n - 1, C * r))}[change]
+        bad[i] = t
+        try:
+            layer_ops.mcmoe_coef(*bad, 4, C)
+        except (RuntimeError, ValueError):   # the torch ops' refusal
+            assert change != "sigma type"
+        else:
+            assert change == "sigma type"
+    assert taken == ["kernel"]
+
+
+def test_mcmoe_router_of_another_size_is_refused():
+    """As ever: the coefficients have the module's components, whatever the router gives."""
+    from verace_amd import ManifoldContinuousMoE
+    m = ManifoldContinuousMoE(D, rank=8, num_components=16, top_k_components=4)
+    m.router = nn.Linear(D, 8, bias=False)
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        m(torch.randn(2, 3, D))
+
+
 class _Lib:
     """Every entry point of the library, doing nothing."""
 

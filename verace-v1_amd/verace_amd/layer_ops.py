@@ -135,7 +135,8 @@ def norm_add(a: torch.Tensor, norm1=None, c: Optional[torch.Tensor] = None,
 
 def situ_glu(g: torch.Tensor, u: torch.Tensor, beta1: float, beta2: float) -> torch.Tensor:
     """``[b1 tanh(g / b1) sigmoid(g)] * [b2 tanh(u / b2)]``."""
-    if (fusable(g) and isinstance(beta1, (int, float)) and isinstance(beta2, (int, float)) and type(u) is torch.Tensor and u.dtype == g.dtype and u.shape == g.shape
+    if (fusable(g) and isinstance(beta1, (int, float)) and isinstance(beta2, (int, float))
+            and type(u) in _PLAIN and u.dtype == g.dtype and u.device == g.device and u.shape == g.shape
             and g.numel() > 0 and g.numel() % (16 // g.dtype.itemsize) == 0 and _rows(g, u)):
         out = torch.empty_like(g)
         _lib.check(_lib.load().vmi_situ_glu(_ptr(g), _ptr(u), _lib.dtype_code(g.dtype), beta1, beta2,
@@ -145,14 +146,18 @@ def situ_glu(g: torch.Tensor, u: torch.Tensor, beta1: float, beta2: float) -> to
     return (beta1 * torch.tanh(g / beta1) * torch.sigmoid(g)) * (beta2 * torch.tanh(u / beta2))
 
 
-def mcmoe_coef(logits: torch.Tensor, sig: torch.Tensor, vproj: torch.Tensor, top_k: int) -> torch.Tensor:
-    """``vproj * sigmoid(sig) * weight`` [n, C * r] with the weights the softmax over the top-k
-    logits (keep-top-k before the softmax, mcmoe.py:82-87), 0 off the top k."""
-    n, C = logits.shape
+def mcmoe_coef(logits: torch.Tensor, sig: torch.Tensor, vproj: torch.Tensor, top_k: int,
+               components: Optional[int] = None) -> torch.Tensor:
+    """``vproj * sigmoid(sig) * weight`` [n, C * r] of C = ``components`` (by default as many as
+    logits), with the weights the softmax over the top-k logits (keep-top-k before the softmax,
+    mcmoe.py:82-87), 0 off the top k."""
+    n = logits.shape[0]
+    C = logits.shape[1] if components is None else components
     r = vproj.shape[1] // C
-    if (fusable(logits) and all(type(t) is torch.Tensor and t.dtype == logits.dtype for t in (sig, vproj))
-            and n > 0 and C <= 64 and r <= 4096 and r % (16 // logits.dtype.itemsize) == 0
-            and sig.shape == vproj.shape and _rows(sig, vproj) and logits.is_contiguous()):
+    if (fusable(logits) and all(type(t) in _PLAIN and t.dtype == logits.dtype and t.device == logits.device
+                                and tuple(t.shape) == (n, C * r) for t in (sig, vproj))
+            and tuple(logits.shape) == (n, C) and n > 0 and 1 <= top_k <= C <= 64 and 0 < r <= 4096
+            and r % (16 // logits.dtype.itemsize) == 0 and _rows(sig, vproj) and logits.is_contiguous()):
         coef = torch.empty_like(vproj)
         _lib.check(_lib.load().vmi_mcmoe_coef(_ptr(logits), _ptr(sig), _ptr(vproj),
                                               _lib.dtype_code(logits.dtype), top_k, _ptr(coef), n, C, r,

@@ -62,7 +62,7 @@ class ManifoldContinuousMoE(nn.Module):
         base_out = self.base_w_down(self.base_situ_glu(xf))
         # v_proj[n, j, :] = V_j x_n for every component, then the selected ones' coefficients
         vproj = xf @ self.v_basis.reshape(C * r, d).t()
-        coef = mcmoe_coef(self.router(xf), self.hyper_sigma(xf), vproj, min(self.top_k_components, C))
+        coef = mcmoe_coef(self.router(xf), self.hyper_sigma(xf), vproj, min(self.top_k_components, C), C)
         return base_out, coef @ self.u_basis.permute(0, 2, 1).reshape(C * r, d)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
