@@ -63,3 +63,26 @@ def test_unit_rows_double_backward(device):
         g, = torch.autograd.grad((f(x) * w).sum(), x, create_graph=True)
         out.append(torch.autograd.grad(g.pow(2).sum(), x)[0])
     assert torch.allclose(out[0], out[1], rtol=1e-4, atol=1e-5)
+
+
+def test_unit_rows_observed(device):
+    """A function mode, a trace and a compiler see F.normalize's ops, in the CHAM projections too."""
+    from torch.overrides import TorchFunctionMode
+    from verace_amd import ContinuousHolographicMemory
+    from verace_amd.hip_kernels import unit_rows
+    seen = []
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    x = torch.randn(3, 8, device=device)
+    ref = F.normalize(x, p=2, dim=-1)
+    m = ContinuousHolographicMemory(16, 32).to(device)
+    with torch.no_grad(), Watch():
+        y = unit_rows(x)
+        m.project(torch.randn(1, 2, 16, device=device))
+    assert seen.count(F.normalize) == 4 and torch.equal(y, ref)
+    traced = torch.jit.trace(unit_rows, x)
+    assert "PythonOp" not in str(traced.graph) and torch.equal(traced(2 * x), F.normalize(2 * x, p=2, dim=-1))
+    assert torch.equal(torch.compile(unit_rows, backend="eager", fullgraph=True)(x), ref)

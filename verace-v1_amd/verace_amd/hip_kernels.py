@@ -228,18 +228,26 @@ class UnitRowsFunction(torch.autograd.Function):
         return dx, None
 
 
-def unit_rows(x: torch.Tensor) -> torch.Tensor:
-    """``F.normalize(x, p=2, dim=-1)``, on the fused kernels for plain device tensors that autograd
-    differentiates.  Under autocast the result of 16-bit rows is fp32, as F.normalize's; fp16 rows
-    without autocast keep its op sequence (there eps rounds to zero)."""
-    out = torch.float32 if torch.is_autocast_enabled("cuda") else x.dtype
-    if (type(x) is torch.Tensor and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
-            and (x.dtype, out) != (torch.float16, torch.float16) and 1 <= x.shape[-1] <= 1024
-            and 0 < x.numel() // x.shape[-1] < 2 ** 31 and x.is_contiguous()
-            and torch._C._functorch.peek_interpreter_stack() is None
+def unobserved() -> bool:
+    """Whether no tracing, functorch transform, forward-mode AD or dispatch / function mode sees the ops
+    that run now, so that kernels outside torch's dispatcher may take their place."""
+    return (not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and torch.autograd.forward_ad._current_level < 0
-            and torch._C._len_torch_dispatch_stack() == 0):
-        return UnitRowsFunction.apply(x, out)
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0)
+
+
+def unit_rows(x: torch.Tensor) -> torch.Tensor:
+    """``F.normalize(x, p=2, dim=-1)``, on the fused kernels for plain device tensors while nothing
+    observes its ops.  Under autocast the result of 16-bit rows is fp32, as F.normalize's; fp16 rows
+    without autocast keep its op sequence (there eps rounds to zero)."""
+    if (unobserved() and type(x) is torch.Tensor and x.is_cuda
+            and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and 1 <= x.shape[-1] <= 1024
+            and 0 < x.numel() // x.shape[-1] < 2 ** 31 and x.is_contiguous()):
+        out = torch.float32 if torch.is_autocast_enabled("cuda") else x.dtype
+        if (x.dtype, out) != (torch.float16, torch.float16):
+            return UnitRowsFunction.apply(x, out)
     return torch.nn.functional.normalize(x, p=2, dim=-1)
 
 

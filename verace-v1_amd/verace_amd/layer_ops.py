@@ -14,11 +14,10 @@ from typing import Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
 from . import _lib
-from .hip_kernels import rms_default_eps
+from .hip_kernels import rms_default_eps, unobserved
 
 _DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
@@ -30,12 +29,7 @@ def _ptr(t):
 def fusable(x: torch.Tensor) -> bool:
     """Whether kernels outside torch's dispatcher may take this tensor's place in the op sequence."""
     return (type(x) is torch.Tensor and x.is_cuda and x.dtype in _DTYPES and not torch.is_grad_enabled()
-            and not torch.is_autocast_enabled("cuda")
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and forward_ad._current_level < 0
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._len_torch_function_stack() == 0)
+            and not torch.is_autocast_enabled("cuda") and unobserved())
 
 
 def plain(m, cls) -> bool:
