@@ -81,6 +81,24 @@ def test_mcmoe_coef_nonfinite_logits(device):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_mcmoe_coef_nonfinite_off_the_top_k(device, dtype):
+    """Infinite and NaN projections and sigmas of components off the top k give NaN, as the torch
+    ops' product with a weight of 0 does, in their own place alone."""
+    from verace_amd.layer_ops import mcmoe_coef
+    n, C, r, inf = 3, 16, 8, float("inf")
+    logits = torch.arange(C, device=device).flip(0).expand(n, C).to(dtype).contiguous()   # 0 .. 3 kept
+    sig, v = torch.zeros(n, C * r, device=device, dtype=dtype), torch.ones(n, C * r, device=device, dtype=dtype)
+    v[0, 2 * r], v[0, 9 * r + 1], v[1, 15 * r + 7] = inf, -inf, float("nan")
+    sig[1, 8 * r], sig[2, 5 * r + 2], sig[2, 6 * r], sig[2, 7 * r] = float("nan"), float("nan"), inf, -inf
+    with torch.no_grad():
+        y = mcmoe_coef(logits, sig, v, 4)
+    with torch.enable_grad():   # the torch ops
+        ref = mcmoe_coef(logits, sig, v, 4)
+    assert int(torch.isnan(ref).sum()) == 4
+    assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,d", [(1, 8), (3, 1024), (67, 1032), (2, 4096)])
 @pytest.mark.parametrize("which", ["norm", "add_norm", "norm_add_norm", "norm_add_add"])
 def test_norm_add(device, dtype, rows, d, which):

@@ -79,12 +79,11 @@ __global__ __launch_bounds__(256) void situ_glu_kernel(const T* __restrict__ g, 
 // ------------------------------------------------------------------ M-CMoE routing
 // Lane = component (C <= 64): weights = softmax over the top-k logits (equal
 // logits by lowest index, as torch.topk takes them), 0 elsewhere; coef[c][j] = vproj[c][j]
-// sigmoid(sig[c][j]) weight[c].  Components off the top k are written as zeros without reading
-// their vproj and sig rows (at k = 8 of 64 that is 7/8 of the input) unless a weight is not finite
-// (a NaN or infinite logit), where the whole row takes 0 or NaN from the same products.
+// sigmoid(sig[c][j]) weight[c].  Components off the top k are read and multiplied like the others: an
+// infinite or NaN vproj or sig there gives NaN, as the tensor ops' product with a weight of 0 does.
 // Four waves share a token's row, the first forms the weights.  (One wave per token with ds_bpermute
-// ranks: 17 us for 64 tokens and 32 us for 8192 at C 64, r 32; all four waves ranking: 10 and 57; so 5
-// and 24.)
+// ranks: 17 us for 64 tokens and 32 us for 8192 at C 64, r 32 bf16; all four waves ranking: 10 and 57;
+// so 5 and 27.)
 constexpr int GW = 4;  // waves per token
 template <typename T>
 __global__ __launch_bounds__(64 * GW) void mcmoe_coef_kernel(const T* __restrict__ logits,
@@ -116,8 +115,7 @@ __global__ __launch_bounds__(64 * GW) void mcmoe_coef_kernel(const T* __restrict
     float sum = p;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
-    // 0 off the top k; NaN throughout if the sum is not finite.  -1 marks a component not to read.
-    ws[lane] = sel || !(sum < __builtin_inff()) ? p / sum : -1.f;
+    ws[lane] = p / sum;  // 0 off the top k; NaN throughout if the sum is not finite
   }
   __syncthreads();
   constexpr int N = Vec<T>::N;
@@ -125,13 +123,11 @@ __global__ __launch_bounds__(64 * GW) void mcmoe_coef_kernel(const T* __restrict
   for (int e = threadIdx.x; e < total; e += 64 * GW) {
     const float wc = ws[e / per];
     const int64_t o = t * C * r + static_cast<int64_t>(e) * N;
-    Vec<T> y = {};
-    if (!(wc < 0.f)) {
-      const Vec<T> s = ldv(sig + o), v = ldv(vproj + o);
+    const Vec<T> s = ldv(sig + o), v = ldv(vproj + o);
+    Vec<T> y;
 #pragma unroll
-      for (int j = 0; j < N; ++j)
-        y.e[j] = round_to<T>(io<T>::to_f32(v.e[j]) * sigmoid_for<T>(io<T>::to_f32(s.e[j])) * wc);
-    }
+    for (int j = 0; j < N; ++j)
+      y.e[j] = round_to<T>(io<T>::to_f32(v.e[j]) * sigmoid_for<T>(io<T>::to_f32(s.e[j])) * wc);
     stv(coef + o, y);
   }
 }
