@@ -152,6 +152,35 @@ def test_halting_updates_match_torch(device, dtype, b, s, d):
     assert 0 < int((ref[1] < 6).sum()) or b * s == 1
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("where", ["bias", "weight", "token", "infinite token", "infinite weight"])
+def test_halting_updates_nonfinite(device, dtype, where):
+    """NaN and infinite halting inputs and tokens: final states, depths and activity are NaN exactly
+    where the torch ops make them so, whether the token is active, halts or has halted."""
+    from verace_amd import AdaptiveCognitiveDepthEngine
+    torch.manual_seed(3)
+    d = 64
+    eng = AdaptiveCognitiveDepthEngine(d, 0.9).to(device, dtype)
+    with torch.no_grad():
+        eng.w_halting.weight.copy_(torch.randn(1, d) / d ** 0.5)
+        x = torch.randn(4, 3, d, device=device).to(dtype)
+        bad = float("inf") if where.startswith("infinite") else float("nan")
+        if where == "bias":
+            eng.w_halting.bias.fill_(bad)
+        elif where.endswith("weight"):
+            eng.w_halting.weight[0, 5] = bad
+        else:
+            x[1, 2, 7] = bad
+        layers = [_Shift(device, dtype, d, i) for i in range(4)]
+        eng_ref = _TorchEngine(eng, d).to(device, dtype)
+        got = eng.run(layers, x, 4, 1, step_states=_States(4), static_control=True)
+        ref = eng_ref.run(layers, x, 4, 1, step_states=_States(4), static_control=True)
+    for a, b in zip(got[:2], ref[:2]):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
+    if where in ("bias", "weight"):
+        assert torch.isnan(ref[1]).all()
+
+
 class _Shift(nn.Module):
     def __init__(self, device, dtype, d, i):
         super().__init__()

@@ -219,11 +219,12 @@ __global__ __launch_bounds__(NTH) void norm_add_kernel(const T* __restrict__ a, 
 // One adaptive-depth step of every token (acd_engine.py:128-150), one workgroup per token, all
 // quantities rounded to the stream's type after each operation as the tensor ops are:
 //   h' = active ? out : h;  p = sigmoid(w . h' + b) (0 below the minimum depth);  acc' = acc + p;
-//   halted = active and acc' >= threshold;  rem = max(1 - acc, 0);
-//   final += (halted ? rem : active ? p : 0) h';  depth += active, then + rem where halted;
-//   active' = active and not halted.
-// mode: 0 as above, 1 below the minimum depth (p = 0), 2 the loop's end: the tokens still active add
-// rem h to final and rem to depth, and nothing else changes.
+//   halted = active and acc' >= threshold;  rem = 1 - acc, 0 where that is negative (NaN kept);
+//   final += ((halted ? rem : p) active) h';  depth += active, then += rem halted;
+//   active' = active and not halted
+// (active and halted as 0 or 1: a NaN p or rem reaches the sums of every token, as in the tensor ops).
+// mode: 0 as above, 1 below the minimum depth (p = 0), 2 the loop's end: final += (rem active) h,
+// depth += rem active, and nothing else changes.
 template <typename T>
 __global__ __launch_bounds__(NTH) void halting_kernel(const T* out, const T* h, T* h_next,
                                                       const T* __restrict__ w, const T* __restrict__ bias,
@@ -254,8 +255,8 @@ __global__ __launch_bounds__(NTH) void halting_kernel(const T* out, const T* h, 
   const float p = mode == 0 ? rounded<T>(sigmoid_for<float>(rounded<T>(dot + io<T>::load(bias, 0)))) : 0.f;
   const float a1 = rounded<T>(a0 + p);
   const bool halted = on && (mode == 2 || a1 >= threshold);
-  const float rem = fmaxf(rounded<T>(1.f - a0), 0.f);
-  const float wt = on ? (halted ? rem : p) : 0.f;
+  const float left = rounded<T>(1.f - a0), rem = left < 0.f ? 0.f : left;
+  const float wt = (halted ? rem : p) * (on ? 1.f : 0.f);
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int i = threadIdx.x + NTH * v;
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(NTH) void halting_kernel(const T* out, const T* h, 
   }
   if (threadIdx.x == 0) {
     float dn = mode == 2 ? dp : rounded<T>(dp + (on ? 1.f : 0.f));
-    dn = rounded<T>(dn + (halted ? rem : 0.f));
+    dn = rounded<T>(dn + rem * (halted ? 1.f : 0.f));
     io<T>::store(depth, t, dn);
     if (mode == 2) return;
     io<T>::store(acc, t, a1);
