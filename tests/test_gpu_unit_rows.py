@@ -86,3 +86,25 @@ def test_unit_rows_observed(device):
     traced = torch.jit.trace(unit_rows, x)
     assert "PythonOp" not in str(traced.graph) and torch.equal(traced(2 * x), F.normalize(2 * x, p=2, dim=-1))
     assert torch.equal(torch.compile(unit_rows, backend="eager", fullgraph=True)(x), ref)
+
+
+def test_replaced_project_runs_in_training(device):
+    """A subclass's or an instance's own ``project(x, active_mask)`` is called as in inference."""
+    from verace_amd import SSSDAttention
+    calls = []
+
+    class Own(SSSDAttention):
+        def project(self, x, active_mask=None):
+            calls.append(active_mask)
+            return super().project(x, active_mask)
+    torch.manual_seed(0)
+    a, b = Own(64, 2, 16).to(device), SSSDAttention(64, 2, 16).to(device)
+    b.load_state_dict(a.state_dict())
+    x = torch.randn(2, 5, 64, device=device, requires_grad=True)
+    mask = torch.ones(2, 5, device=device, dtype=torch.bool)
+    ya, yb = a(x, active_mask=mask)[0], b(x, active_mask=mask)[0]
+    assert len(calls) == 1 and calls[0] is mask and torch.allclose(ya, yb, rtol=1e-4, atol=1e-5)
+    plain = b.project
+    b.project = lambda x, active_mask=None: calls.append(b) or plain(x, active_mask)
+    b(x)[0].sum().backward()
+    assert calls[-1] is b and bool(x.grad.isfinite().all())

@@ -95,10 +95,12 @@ class SSSDAttention(nn.Module):
         return launch_sssd_hip_scan_fused(proj, self.num_heads, self.head_dim, active_mask,
                                           w.detach(), self.head_rmsnorm.eps, initial_state)
 
-    def project(self, x: torch.Tensor, active_mask: Optional[torch.Tensor] = None,
-                norm=partial(F.normalize, p=2, dim=-1)):
-        """q, k, v [B,T,H,D] (L2-normalised, by ``norm``) and delta [B,T,H] as the reference builds
-        them (``sssd_attention.py:116-126``)."""
+    def project(self, x: torch.Tensor, active_mask: Optional[torch.Tensor] = None):
+        """q, k, v [B,T,H,D] (L2-normalised) and delta [B,T,H] as the reference builds them
+        (``sssd_attention.py:116-126``)."""
+        return self._project(x, active_mask, partial(F.normalize, p=2, dim=-1))
+
+    def _project(self, x, active_mask, norm):
         b, s, _ = x.shape
         H, D = self.num_heads, self.head_dim
         q, k, v = (norm(w(x).view(b, s, H, D)) for w in (self.w_q, self.w_k, self.w_v))
@@ -132,7 +134,10 @@ class SSSDAttention(nn.Module):
         rms_grad = (torch.is_grad_enabled() and self.head_rmsnorm.weight is not None
                     and self.head_rmsnorm.weight.requires_grad)
         if grad:
-            q, k, v, delta = self.project(x, active_mask, unit_rows)
+            if type(self).project is SSSDAttention.project and "project" not in self.__dict__:
+                q, k, v, delta = self._project(x, active_mask, unit_rows)
+            else:  # a replaced method
+                q, k, v, delta = self.project(x, active_mask)
             o, psi = sssd_scan(q, k, v, delta, initial_state)
             o_norm = self.head_rmsnorm(o).view(b, s, self.num_heads * self.head_dim)
         elif self._fused(x):
