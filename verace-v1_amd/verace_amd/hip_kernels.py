@@ -198,7 +198,7 @@ _UNIT_EPS = 1e-12  # F.normalize's default
 
 class UnitRowsFunction(torch.autograd.Function):
     """``F.normalize(x, dim=-1)`` of contiguous rows in one kernel each way; the result in
-    ``out_dtype``.  A backward that is itself differentiated runs the torch ops."""
+    ``out_dtype``.  A backward that is itself differentiated is F.normalize's."""
 
     @staticmethod
     def forward(ctx, x, out_dtype):
@@ -215,9 +215,9 @@ class UnitRowsFunction(torch.autograd.Function):
         x, = ctx.saved_tensors
         if torch.is_grad_enabled():  # create_graph
             with torch.autocast("cuda", enabled=False):
-                n = torch.linalg.vector_norm(x.to(dy.dtype), dim=-1, keepdim=True).clamp_min(_UNIT_EPS)
-                y = x.to(dy.dtype) / n
-                return ((dy - y * (y * dy).sum(-1, keepdim=True)) / n).to(x.dtype), None
+                x = x.view_as(x)  # without x's own hooks: they run on what this returns
+                y = torch.nn.functional.normalize(x.to(dy.dtype), p=2, dim=-1)
+                return torch.autograd.grad(y, x, dy, create_graph=True)[0], None
         dy = dy.contiguous()
         dx = torch.empty_like(x)
         D = x.shape[-1]
