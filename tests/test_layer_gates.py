@@ -112,6 +112,20 @@ def test_mcmoe_router_of_another_size_is_refused():
         m(torch.randn(2, 3, D))
 
 
+def test_plain_modules_only():
+    """A module compiled in place runs its compiled call, as one with hooks or another forward does."""
+    assert layer_ops.plain(nn.Linear(4, 4), nn.Linear)
+    m = nn.Linear(4, 4)
+    m.compile(backend="eager")
+    assert not layer_ops.plain(m, nn.Linear)
+    m = nn.Linear(4, 4)
+    m.register_forward_pre_hook(lambda *a: None)
+    assert not layer_ops.plain(m, nn.Linear)
+    m = nn.Linear(4, 4)
+    m.forward = lambda x: x
+    assert not layer_ops.plain(m, nn.Linear)
+
+
 class _Lib:
     """Every entry point of the library, doing nothing."""
 

@@ -36,7 +36,8 @@ def plain(m, cls) -> bool:
     """A module of exactly ``cls`` whose call does no more than its own ``forward``."""
     return (type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks
             and not m._backward_hooks and not m._backward_pre_hooks
-            and "forward" not in m.__dict__ and not _module._has_any_global_hook())
+            and "forward" not in m.__dict__ and m._compiled_call_impl is None
+            and not _module._has_any_global_hook())
 
 
 def _rows(*ts) -> bool:
