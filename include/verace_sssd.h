@@ -84,8 +84,9 @@ int vmi_sssd_scan_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D,
  * Supported: io_dtype in {F32, BF16, F16}; delta_dtype in {F32, BF16, F16};
  * 1 <= D <= 256.  T = 0 copies psi_in (or identity) to psi_out.
  * Arithmetic: F32 I/O, D != 128 and T < 32 run in fp32: in chunks of 16 tokens on the fp32
- * matrix cores for 5 <= T and D <= 128, given the workspace of vmi_sssd_scan_workspace_bytes
- * (optional for these calls: without it, or with less, they run token by token, as T < 5,
+ * matrix cores for D <= 128 and T >= 5 (up to 20 for small D and many heads, where fewer tokens are
+ * faster one by one), given the workspace of vmi_sssd_scan_workspace_bytes (0 for the others;
+ * optional for these: without it, or with less, they run token by token, as fewer tokens,
  * D > 128 and any sequence with a non-finite token or one of ((delta / 2) |k| |v|)^2 > 0.003
  * always do: past that bound the chunk form would round worse than the token-by-token one; unit
  * k, v with delta <= 0.1 stay below 0.0026).

@@ -63,6 +63,21 @@ def test_workspace_query(lib):
     assert lib.vmi_cham_scan_workspace_bytes(1, 64, 1025, ctypes.byref(n)) == 2
 
 
+@pytest.mark.parametrize("BH,D,least", [(1, 128, 5), (4096, 65, 5), (512, 64, 5), (513, 64, 9), (1, 33, 5),
+                                        (16, 32, 5), (17, 32, 6), (32, 32, 6), (33, 16, 7), (128, 32, 8), (225, 4, 10),
+                                        (65536, 32, 10), (1, 30, 8), (129, 7, 20)])
+def test_short_fp32_scans_run_token_by_token(lib, BH, D, least):
+    """The chunked fp32 scan (the one that asks for workspace) takes calls from the length on at which
+    it is the faster."""
+    n = ctypes.c_size_t(0)
+    for T in range(1, 25):
+        assert lib.vmi_sssd_scan_workspace_bytes(1, T, BH, D, 0, ctypes.byref(n)) == 0
+        assert (n.value > 0) == (T >= least), T
+    if D <= 32 and least < 20:   # 16-bit rows: later
+        assert lib.vmi_sssd_scan_workspace_bytes(1, least, BH, D, 1, ctypes.byref(n)) == 0 and n.value == 0
+    assert lib.vmi_sssd_scan_workspace_bytes(1, 64, BH, 129, 0, ctypes.byref(n)) == 0 and n.value == 0
+
+
 def test_argument_errors_before_any_device_call(lib):
     # null pointers / bad sizes are rejected on the host (no HIP call is made)
     assert lib.vmi_sssd_scan_fwd(None, None, None, None, 1, 1, None, None, None,

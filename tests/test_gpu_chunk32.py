@@ -72,7 +72,7 @@ def _slice_err(x, ref, dims):
 # rows that are not whole 16-byte pieces, and sequences long enough for several segments
 SHAPES = [(1, 5, 1, 1), (1, 8, 2, 128), (2, 15, 2, 15), (1, 16, 3, 16), (2, 17, 1, 17), (1, 31, 2, 32),
           (1, 33, 2, 33), (2, 48, 2, 63), (1, 129, 2, 64), (2, 20, 3, 65), (1, 50, 2, 100),
-          (1, 40, 2, 127), (2, 100, 2, 128), (1, 1030, 2, 128), (2, 999, 1, 40), (3, 700, 3, 30)]
+          (1, 9, 1, 1), (1, 7, 2, 16), (1, 5, 2, 33), (1, 5, 1, 65), (1, 40, 2, 127), (2, 100, 2, 128), (1, 1030, 2, 128), (2, 999, 1, 40), (3, 700, 3, 30)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])

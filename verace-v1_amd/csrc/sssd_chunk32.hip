@@ -664,10 +664,30 @@ hipError_t launch_io(const Plan& pl, const void* q, const void* k, const void* v
 
 }  // namespace c32
 
-bool use_chunk32(int64_t T, int64_t D) { return T >= kChunk32MinT && D <= 128; }
+// Up to 16 tokens are one chunk: four launches whose time is that of filling the chip, where the
+// token-sequential scan takes one launch and 2.3 / 3 / 6 us a token at head_dim 32 / 64 / 128.  Both in us
+// (fp32, chunk / sequential):
+//   D 128: T 5 BH 4 20 / 35, BH 4096 205 / 359: the chunk from 5 tokens on at any number of heads;
+//   D 64:  T 5 BH 512 19 / 22, BH 2048 46 / 38; T 9 BH 2048 46 / 57 (D 33 bf16, rows unaligned, 53 / 56);
+//   D 32:  the chunk's time grows with the heads already below a full chip: T 6 BH 32 15 / 17, BH 128
+//          20 / 17; T 8 BH 128 20 / 22, BH 256 26 / 22; T 10 BH 256 26 / 27, BH 4096 55 / 57.  16-bit
+//          rows take 1.5 more (T 9 BH 192 25.5 / 24.7, T 5 BH 16 15.0 / 14.1), and rows that are not
+//          whole 4-element pieces more again (D 7 T 7 BH 64 21 / 19; bf16 T 17 BH 4096 96 / 86).
+int64_t chunk32_min_tokens(int64_t BH, int64_t D, int io_dtype) {
+  if (D > 64) return 5;
+  if (D > 32) return BH <= 512 ? 5 : 9;
+  const bool f32 = io_dtype == VMI_F32, pieces = D % 4 == 0;
+  if (BH <= 16 && f32 && pieces) return 5;
+  if (BH > 128 && !pieces) return 20;
+  return std::min<int64_t>(10, 6 + (BH + 31) / 64) + (f32 ? 0 : 1) + (pieces ? 0 : 2);
+}
 
-size_t chunk32_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D) {
-  if (!use_chunk32(T, D) || B <= 0 || H <= 0) return 0;
+bool use_chunk32(int64_t BH, int64_t T, int64_t D, int io_dtype) {
+  return D <= 128 && T >= chunk32_min_tokens(BH, D, io_dtype);
+}
+
+size_t chunk32_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D, int io_dtype) {
+  if (B <= 0 || H <= 0 || !use_chunk32(B * H, T, D, io_dtype)) return 0;
   return c32::plan(B, T, H, D).total;
 }
 

@@ -1,8 +1,9 @@
 // Token-sequential SSSD scan, fp32 arithmetic, one workgroup per (batch, head).
 //
-// This is the path for head_dim above 128, single tokens at head_dim other than 128, calls
-// without workspace and the sequences a chunk scan flagged as outside its accuracy envelope.  The state Psi (D x D fp32) lives in VGPRs for
-// the whole scan: thread (rg, cg) owns rows {rg + RG*m} and the four columns
+// This is the path for head_dim above 128, calls of few tokens (below chunk32_min_tokens; single
+// ones at head_dim 128 have sssd_step.hip), calls without workspace and the sequences a chunk scan
+// flagged as outside its accuracy envelope.  The state Psi (D x D fp32) lives in VGPRs for the whole
+// scan: thread (rg, cg) owns rows {rg + RG*m} and the four columns
 // 4cg..4cg+3, so loads and stores of Psi are float4 and fully coalesced.
 //
 // Per token t (reference: sssd_attention.py:160-175, applied one step at a

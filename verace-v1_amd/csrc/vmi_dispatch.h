@@ -112,13 +112,11 @@ hipError_t launch_sssd_seq(const void* q, const void* k, const void* v, const vo
                            float* psi_out, int B, int T, int H, int D, hipStream_t stream,
                            const FlaggedSegments& map);
 
-// sssd_chunk32.hip: chunked scan in fp32 (any I/O dtype, head_dim <= 128).
-// Below 5 tokens the token-sequential kernel is the shorter (one launch, about 4 us a token at
-// head_dim 64: 10 us at T = 2, 19.6 us at T = 5, against 16 us here for any T <= 16) and rounds no
-// more.
-constexpr int64_t kChunk32MinT = 5;
-bool use_chunk32(int64_t T, int64_t D);
-size_t chunk32_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D);
+// sssd_chunk32.hip: chunked scan in fp32 (any I/O dtype, head_dim <= 128), from chunk32_min_tokens
+// on; shorter calls are shorter token by token and round no more.
+int64_t chunk32_min_tokens(int64_t BH, int64_t D, int io_dtype);
+bool use_chunk32(int64_t BH, int64_t T, int64_t D, int io_dtype);
+size_t chunk32_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D, int io_dtype);
 hipError_t launch_sssd_chunk32(const void* q, const void* k, const void* v, const void* delta,
                                int io_dtype, int delta_dtype, const float* psi_in, void* out,
                                float* psi_out, int B, int T, int H, int D, void* workspace,
