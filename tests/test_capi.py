@@ -78,6 +78,16 @@ def test_short_fp32_scans_run_token_by_token(lib, BH, D, least):
     assert lib.vmi_sssd_scan_workspace_bytes(1, 64, BH, 129, 0, ctypes.byref(n)) == 0 and n.value == 0
 
 
+def test_fp32_scans_beyond_a_launch_run_token_by_token(lib):
+    """The chunked fp32 scan's launches hold fewer than 2^32 threads: 128 a head at D = 32, 64 a chunk."""
+    n = ctypes.c_size_t(0)
+    for T, BH, D, chunked in ((16, 33_000_000, 32, True), (16, 34_000_000, 32, False), (12, 8_388_607, 128, True),
+                              (12, 8_388_608, 128, False), (1_000_000_000, 1, 4, True),
+                              (2_000_000_000, 1, 4, False), (64, 17_000_000, 4, False)):
+        assert lib.vmi_sssd_scan_workspace_bytes(1, T, BH, D, 0, ctypes.byref(n)) == 0
+        assert (n.value > 0) == chunked, (T, BH, D)
+
+
 def test_argument_errors_before_any_device_call(lib):
     # null pointers / bad sizes are rejected on the host (no HIP call is made)
     assert lib.vmi_sssd_scan_fwd(None, None, None, None, 1, 1, None, None, None,

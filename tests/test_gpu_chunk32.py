@@ -158,6 +158,26 @@ def test_chunk32_never_rounds_worse_than_the_sequential_scan(device, length, ang
             assert e <= 2.0 * es + 2e-7
 
 
+def test_scan_without_room_for_its_workspace(device, monkeypatch):
+    """The fp32 scan, whose workspace is optional, runs without it where its allocation fails; the
+    16-bit chunk scan, which needs its own, raises that failure."""
+    from verace_amd import launch_sssd_hip_scan
+    empty = torch.empty
+
+    def no_bytes(*args, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*args, **kw)
+    q, k, v, delta, psi0 = _inputs(1, 600, 2, 64, torch.float32, 11)
+    ref = _c_scan(q, k, v, delta, psi0, device, workspace=False)
+    monkeypatch.setattr(torch, "empty", no_bytes)
+    o, psi = launch_sssd_hip_scan(*(t.to(device) for t in (q, k, v, delta, psi0)))
+    assert torch.equal(o.cpu(), ref[0]) and torch.equal(psi.cpu(), ref[1])
+    q, k, v, delta, _ = _inputs(1, 600, 2, 128, torch.bfloat16, 12)
+    with pytest.raises(torch.OutOfMemoryError):
+        launch_sssd_hip_scan(*(t.to(device) for t in (q, k, v, delta)))
+
+
 def test_chunk32_wide_and_nonfinite_sequences_take_the_sequential_scan(device):
     """A sequence with a token above the chunk form's limit, or one whose Cayley factor
     is not finite, gives the token-sequential scan's bits; the others the chunk result."""

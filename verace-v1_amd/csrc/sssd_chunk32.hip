@@ -683,7 +683,12 @@ int64_t chunk32_min_tokens(int64_t BH, int64_t D, int io_dtype) {
 }
 
 bool use_chunk32(int64_t BH, int64_t T, int64_t D, int io_dtype) {
-  return D <= 128 && T >= chunk32_min_tokens(BH, D, io_dtype);
+  // a launch holds fewer than 2^32 threads: 64 per chunk in the preparation, 4 per padded feature and
+  // sequence in the passes (one segment then; the sequential kernel's are no more)
+  constexpr int64_t kThreads = int64_t(1) << 32;
+  const int64_t dp = D <= 32 ? 32 : D <= 64 ? 64 : 128;
+  return D <= 128 && T >= chunk32_min_tokens(BH, D, io_dtype) && 4 * dp * BH < kThreads &&
+         (T + c32::C - 1) / c32::C * BH < kThreads / 64 - c32::PW;
 }
 
 size_t chunk32_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t D, int io_dtype) {

@@ -60,6 +60,8 @@ EXPORTED = (
     "vmi_halting_update",
 )
 
+ERR_WORKSPACE = 3  # VMI_ERR_WORKSPACE
+
 _lib = None
 _load_error = None
 

@@ -96,13 +96,18 @@ def launch_sssd_hip_scan(
     ws_bytes = ctypes.c_size_t(0)
     _lib.check(lib.vmi_sssd_scan_workspace_bytes(b, s, h, d_k, io_code, ctypes.byref(ws_bytes)),
                "vmi_sssd_scan_workspace_bytes")
-    ws = None
+    ws, no_room = None, None
     if ws_bytes.value > 0:
-        ws = torch.empty(ws_bytes.value, device=q.device, dtype=torch.uint8)
-    _lib.check(lib.vmi_sssd_scan_fwd(_ptr(q_c), _ptr(k_c), _ptr(v_c), _ptr(delta_c), io_code,
-                                     d_code, _ptr(psi_in), _ptr(out), _ptr(psi_out), b, s, h, d_k,
-                                     _ptr(ws), ws_bytes.value, _lib.stream_handle(q.device)),
-               "vmi_sssd_scan_fwd")
+        try:
+            ws = torch.empty(ws_bytes.value, device=q.device, dtype=torch.uint8)
+        except torch.OutOfMemoryError as e:
+            no_room = e  # the fp32 scans run without theirs
+    status = lib.vmi_sssd_scan_fwd(_ptr(q_c), _ptr(k_c), _ptr(v_c), _ptr(delta_c), io_code, d_code,
+                                   _ptr(psi_in), _ptr(out), _ptr(psi_out), b, s, h, d_k, _ptr(ws),
+                                   0 if ws is None else ws_bytes.value, _lib.stream_handle(q.device))
+    if no_room is not None and status == _lib.ERR_WORKSPACE:
+        raise no_room
+    _lib.check(status, "vmi_sssd_scan_fwd")
     return out, psi_out
 
 
