@@ -787,16 +787,26 @@ __global__ __launch_bounds__(4 * D) void bwdc_pass_kernel(Args a) {
 // products with the exact bf16 operand are exact and accumulated in fp32 (v_mfma_f32_16x16x32_bf16:
 // 3 x 16 cycles for 32 k against 8 x 32 on v_mfma_f32_16x16x4_f32); dO Q^T is one exact product.  The
 // inputs stay bf16 in LDS: rows are read 8 bytes at a time, columns by ds_read_b64_tr_b16.
-// No accumulator passes from a 16x16x32 to a 16x16x16 product: the compiler issues the two back to
-// back, and the second then read the sum before the first had written it (measured: dZ wrong in the
-// one tile where they were adjacent); each keeps its own accumulator and the VALU adds them.
+// No accumulator passes from a 16x16x32 to a 16x16x16 product.  The one build that had such a chain
+// (dZ's two products, adjacent in one tile) gave a wrong dZ in that tile, as if the second had read the
+// sum before the first had written it; why is not known, and the assembly of every kernel of the
+// library has no other chain between products of different shapes.  So the sums of 16x16x32 products
+// have a type of their own (Sum32), which a 16x16x16 product does not take: they leave it through a
+// VALU addition or element by element.
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ s16x8 cat(s16x4 a, s16x4 b) {
   return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
-__device__ __forceinline__ f32x4 mma32(s16x8 a, s16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+struct Sum32 {
+  f32x4 v;
+  __device__ __forceinline__ float operator[](int r) const { return v[r]; }
+};
+__device__ __forceinline__ f32x4 operator+(Sum32 a, Sum32 b) { return a.v + b.v; }
+__device__ __forceinline__ f32x4 operator+(Sum32 a, f32x4 b) { return a.v + b; }
+__device__ __forceinline__ f32x4 operator+(f32x4 a, Sum32 b) { return a + b.v; }
+__device__ __forceinline__ Sum32 mma32(s16x8 a, s16x8 b, Sum32 c) {
+  return Sum32{__builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c.v, 0, 0, 0)};
 }
 __device__ __forceinline__ f32x4 unpack4(s16x4 x) {
   const uint2 w = __builtin_bit_cast(uint2, x);
@@ -890,9 +900,10 @@ __global__ __launch_bounds__(4 * D) void bwdc_pass16_kernel(Args a) {
     fetch(c > c0 ? c - 1 : c);  // past the end the last one again, never committed
     const int ln = MAIN && D == 128 ? opaque(lane) : lane, l16 = ln & 15, g = ln >> 4, colj = 16 * wave + l16;
     // S1 = U^T Psi_e (exact parts), dZ = U^T Lam_e + dX Q^T; two tiles (32 rows) a step
-    f32x4 s1[2], dz[2] = {};
+    f32x4 s1[2], dz[2];
+    Sum32 ul[2] = {};
     {
-      f32x4 ph[2] = {}, pl[2] = {};
+      Sum32 ph[2] = {}, pl[2] = {};
       auto ua = [&](int half, int s) {
         const uint16_t* p = U + (16 * half + l16) * PB + 32 * s + 4 * g;
         return cat(ldsb4(p), ldsb4(p + 16));
@@ -911,8 +922,8 @@ __global__ __launch_bounds__(4 * D) void bwdc_pass16_kernel(Args a) {
         pl[1] = mma32(a1, x.l, pl[1]);
         ph[0] = mma32(a0, x.h, ph[0]);
         ph[1] = mma32(a1, x.h, ph[1]);
-        dz[0] = mma32(a0, y, dz[0]);
-        dz[1] = mma32(a1, y, dz[1]);
+        ul[0] = mma32(a0, y, ul[0]);
+        ul[1] = mma32(a1, y, ul[1]);
         pl[0] = mma32(a0, x.m, pl[0]);
         pl[1] = mma32(a1, x.m, pl[1]);
         __builtin_amdgcn_sched_barrier(0);
@@ -924,8 +935,8 @@ __global__ __launch_bounds__(4 * D) void bwdc_pass16_kernel(Args a) {
     }
     const s16x4 qc = lds_tr(Q, PB, 0, 16 * wave, l16, g);  // tokens 4 g + r of column colj
     const f32x4 none = {0.f, 0.f, 0.f, 0.f};
-    dz[0] += mma_bf16(pack4(lds4(dX + l16 * XPP + 4 * g)), qc, none);
-    dz[1] += mma_bf16(pack4(lds4(dX + (16 + l16) * XPP + 4 * g)), qc, none);
+    dz[0] = ul[0] + mma_bf16(pack4(lds4(dX + l16 * XPP + 4 * g)), qc, none);
+    dz[1] = ul[1] + mma_bf16(pack4(lds4(dX + (16 + l16) * XPP + 4 * g)), qc, none);
     // Wm = T~^T S1, dW = T~^T dZ; MAIN: W = U^T Psi_s = S1 + G Wm, Z = T~ W
     f32x4 wm[2] = {}, dw[2] = {}, w[2], z[2] = {};
 #pragma unroll
@@ -975,7 +986,7 @@ __global__ __launch_bounds__(4 * D) void bwdc_pass16_kernel(Args a) {
       if (S + 1 < SS) nxt = rows(S + 1);
       if constexpr (MAIN) *reinterpret_cast<s16x4*>(LSb + colj * PB + 16 * S + 4 * g) = pack4(lam[S]);
       __builtin_amdgcn_sched_barrier(0);
-      f32x4 d = {}, e = {};
+      Sum32 d = {}, e = {};
       const f32x4 oq = mma_bf16(cur.dv, qc, none);
       d = mma32(cur.u, xw.l, d);
       e = mma32(cur.u, xd.l, e);
@@ -983,7 +994,7 @@ __global__ __launch_bounds__(4 * D) void bwdc_pass16_kernel(Args a) {
       e = mma32(cur.u, xd.m, e);
       d = mma32(cur.u, xw.h, d);
       e = mma32(cur.u, xd.h, e);
-      psi[S] += d;
+      psi[S] = psi[S] + d;
       lam[S] += e + oq;
       if constexpr (MAIN) {
         const s16x4 ps = pack4(psi[S]);
@@ -1009,7 +1020,7 @@ __global__ __launch_bounds__(4 * D) void bwdc_pass16_kernel(Args a) {
       const s16x4 doc = lds_tr(dO, PB, 0, 16 * wave, l16, g);  // dO^T's column colj
       const int half = wave & 1, kp = wave >> 1;               // X: 16 rank rows, columns 32 kp .. + 31
       lds_barrier();  // (1) the column copies visible
-      f32x4 du[2] = {}, du2[2] = {}, dt = {}, x = {};
+      Sum32 du[2] = {}, du2[2] = {}, dt = {}, x = {};
       struct Ops { s16x4 al, ap, z0, z1, w0, w1; };
       auto ops = [&](int kb) {
         return Ops{lds_tr(LSb, PB, 16 * kb, 16 * wave, l16, g), lds_tr(PSb, PB, 16 * kb, 16 * wave, l16, g),
