@@ -238,3 +238,17 @@ def test_fused_steps_stand_aside(device):
         with torch.autocast("cuda", dtype=torch.bfloat16):
             assert not fusable(x)
         assert torch.func.vmap(lambda v: norm_add(v, b=v)[0])(x).shape == x.shape
+
+
+def test_fused_steps_keep_to_the_current_device(device, monkeypatch):
+    """With another device current, as in a program of several, no kernel is launched."""
+    from verace_amd import ManifoldContinuousMoE, _lib
+    from verace_amd.hip_kernels import unit_rows
+    m = ManifoldContinuousMoE(64, rank=8, num_components=16).to(device)
+    x = torch.randn(2, 3, 64, device=device)
+    with torch.no_grad():
+        ref = m(x)
+        monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 1)
+        monkeypatch.setattr(_lib, "load", lambda: pytest.fail("a kernel's entry point was loaded"))
+        assert torch.allclose(m(x), ref, rtol=1e-5, atol=1e-5)
+        assert torch.allclose(unit_rows(x).norm(dim=-1), torch.ones(2, 3, device=device), atol=1e-5)

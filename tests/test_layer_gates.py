@@ -126,6 +126,19 @@ def test_plain_modules_only():
     assert not layer_ops.plain(m, nn.Linear)
 
 
+def test_only_the_current_device(monkeypatch):
+    """Launches go to the current device: tensors of another one keep the torch ops, which run there."""
+    from verace_amd import hip_kernels
+    current = [0]
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current[0])
+    with FakeTensorMode():
+        a, b = torch.empty(2, device="cuda:0"), torch.empty(2, device="cuda:1")
+    assert hip_kernels.on_current_device(a) and not hip_kernels.on_current_device(b)
+    current[0] = 1
+    assert hip_kernels.on_current_device(b) and not hip_kernels.on_current_device(a)
+    assert not hip_kernels.on_current_device(torch.empty(2))
+
+
 class _Lib:
     """Every entry point of the library, doing nothing."""
 

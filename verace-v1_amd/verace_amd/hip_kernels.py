@@ -243,11 +243,17 @@ def unobserved() -> bool:
             and torch._C._len_torch_function_stack() == 0)
 
 
+def on_current_device(x: torch.Tensor) -> bool:
+    """Whether a kernel launched now runs on x's device.  (A launch goes to the calling thread's current
+    device; torch's ops run on their tensors' own.)"""
+    return x.is_cuda and x.get_device() == torch._C._cuda_getDevice()
+
+
 def unit_rows(x: torch.Tensor) -> torch.Tensor:
-    """``F.normalize(x, p=2, dim=-1)``, on the fused kernels for plain device tensors while nothing
-    observes its ops.  Under autocast the result of 16-bit rows is fp32, as F.normalize's; fp16 rows
+    """``F.normalize(x, p=2, dim=-1)``, on the fused kernels for plain tensors of the current device
+    while nothing observes its ops.  Under autocast the result of 16-bit rows is fp32, as F.normalize's; fp16 rows
     without autocast keep its op sequence (there eps rounds to zero)."""
-    if (unobserved() and type(x) is torch.Tensor and x.is_cuda
+    if (unobserved() and type(x) is torch.Tensor and on_current_device(x)
             and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and 1 <= x.shape[-1] <= 1024
             and 0 < x.numel() // x.shape[-1] < 2 ** 31 and x.is_contiguous()):
         out = torch.float32 if torch.is_autocast_enabled("cuda") else x.dtype

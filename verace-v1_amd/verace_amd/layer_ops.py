@@ -2,7 +2,7 @@
 (``csrc/layer_ops.hip``), each beside the torch ops it replaces.
 
 The kernels run where nothing else can be watching the tensors in between: grad mode off, plain
-device tensors of one dtype, no autocast, tracing, functorch transform, forward-mode AD or
+tensors of the current device and of one dtype, no autocast, tracing, functorch transform, forward-mode AD or
 dispatch / function mode, and sub-modules of exactly the expected class without hooks or replaced
 methods.  Everything else takes the torch ops.
 """
@@ -17,7 +17,7 @@ import torch.nn.functional as F
 from torch.nn.modules import module as _module
 
 from . import _lib
-from .hip_kernels import rms_default_eps, unobserved
+from .hip_kernels import on_current_device, rms_default_eps, unobserved
 
 _DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
@@ -28,7 +28,8 @@ def _ptr(t):
 
 def fusable(x: torch.Tensor) -> bool:
     """Whether kernels outside torch's dispatcher may take this tensor's place in the op sequence."""
-    return (type(x) is torch.Tensor and x.is_cuda and x.dtype in _DTYPES and not torch.is_grad_enabled()
+    return (type(x) is torch.Tensor and on_current_device(x) and x.dtype in _DTYPES
+            and not torch.is_grad_enabled()
             and not torch.is_autocast_enabled("cuda") and unobserved())
 
 
