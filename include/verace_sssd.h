@@ -107,8 +107,9 @@ int vmi_sssd_scan_fwd(const void* q, const void* k, const void* v,
 /* The same prefill scan with no workspace argument and no allocation: the scan's workspace
  * is a fixed 40 MiB device array of the library, one per GPU, held from the library's first
  * use on that GPU until the process ends (enough for every plan of the OP, FULL, LONG and DEC
- * shapes; plans needing more return VMI_ERR_WORKSPACE before anything is launched -- use
- * vmi_sssd_scan_fwd for them).  No counterpart in the reference: it is for callers that
+ * shapes; 16-bit D = 128 plans needing more return VMI_ERR_WORKSPACE before anything is launched
+ * -- use vmi_sssd_scan_fwd for them -- and the F32 arithmetic's, optional there, run token by token
+ * without, which is slower by a factor of ten and more: B4 T2048 H8 D128 in F32 is such a call).  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  Calls on one GPU share its array, so calls that overlap on one
  * GPU (several streams or host threads) race: order them.  Arguments and results as

@@ -252,3 +252,27 @@ def test_fused_steps_keep_to_the_current_device(device, monkeypatch):
         monkeypatch.setattr(_lib, "load", lambda: pytest.fail("a kernel's entry point was loaded"))
         assert torch.allclose(m(x), ref, rtol=1e-5, atol=1e-5)
         assert torch.allclose(unit_rows(x).norm(dim=-1), torch.ones(2, 3, device=device), atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_nonfinite_rows(device, dtype):
+    """The activation and the norms are NaN and infinite exactly where the torch ops are."""
+    from verace_amd.layer_ops import norm_add, situ_glu
+    inf, nan, big = float("inf"), float("nan"), torch.finfo(dtype).max
+    g = torch.Generator(device).manual_seed(1)
+    a, b, c = (torch.randn(8, 64, generator=g, device=device).to(dtype) for _ in range(3))
+    for t, vals in ((a, (inf, nan, big, -inf)), (b, (-inf, 1.0, big, inf)), (c, (0.0, 0.0, big, nan))):
+        for r, x in enumerate(vals):
+            t[r, 3 * r] = x
+    n1, n2 = (nn.RMSNorm(64, device=device, dtype=dtype) for _ in range(2))
+
+    def ops():
+        return (situ_glu(a, b, 4.0, 25.0), situ_glu(b, c, 4.0, 25.0), *norm_add(a, b=b, norm2=n2),
+                *norm_add(a, n1, b=b, norm2=n2), norm_add(a, n1, c, b)[0])
+    with torch.no_grad():
+        got = ops()
+    with torch.enable_grad():
+        ref = ops()
+    for i, (x, y) in enumerate(zip(got, ref)):
+        assert torch.equal(torch.isnan(x), torch.isnan(y)) and torch.equal(torch.isinf(x), torch.isinf(y)), i
+    assert any(bool(torch.isnan(y).any()) for y in ref)

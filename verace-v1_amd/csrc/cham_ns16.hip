@@ -36,7 +36,7 @@
 // and load issue.  The wide tile moves half the LDS bytes per product, but one of them fills a CU
 // and [1, 1024, 1024] has 36 and 64 of them: three narrow workgroups share a CU and cover each
 // other's barriers.  Three steps, with 128 x 128 tiles on 4 waves alone before:
-// [1, 1024]^2 455 -> 172 us, [4, 1024]^2 504 -> 485, [4, 512]^2 264 -> 112, [8, 128]^2 96 -> 41.
+// [1, 1024]^2 455 -> 172 us, [4, 1024]^2 511 -> 471, [4, 512]^2 264 -> 112, [8, 128]^2 96 -> 41.
 #include "vmi_common.h"
 #include "vmi_dispatch.h"
 #include "vmi_mfma.h"

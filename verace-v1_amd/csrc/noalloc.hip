@@ -9,7 +9,8 @@
 // kept; the host never passes the array's name to a kernel.  Every call on one GPU shares
 // that GPU's array: calls that overlap on one GPU (two streams, two host threads) race on
 // it, so order them.  The scan's workspace needs no clearing: every part transform and
-// segment start state it holds is written by the scan's first two passes before it is read.
+// segment start state it holds is written by the scan's first two passes before it is read, but for
+// the transforms of segments the fp32 chunk scan flags, whose sequences it runs again.
 #include <mutex>
 
 #include "vmi_common.h"
@@ -64,7 +65,8 @@ extern "C" int vmi_sssd_scan_fwd_noalloc(const void* q, const void* k, const voi
     const char* b = reinterpret_cast<const char*>(psi_out);
     if (a < b + state_bytes && b < a + state_bytes) return VMI_ERR_ALIAS;
   }
-  if (vmi::scan_workspace_required(B, T, H, D, io_dtype) > kScratchBytes) return VMI_ERR_WORKSPACE;  // beyond the fixed array: use vmi_sssd_scan_fwd
+  // beyond the fixed array: use vmi_sssd_scan_fwd
+  if (vmi::scan_workspace_required(B, T, H, D, io_dtype) > kScratchBytes) return VMI_ERR_WORKSPACE;
   if (B == 0 || H == 0) return VMI_OK;
   void* ws = nullptr;
   const size_t want = vmi::scan_workspace_bytes(B, T, H, D, io_dtype);

@@ -3,7 +3,8 @@
 ``VeraceV1Layer`` restates ``verace_v1/modules/backbone.py:21-101`` (same sub-module names,
 order and residual structure: block-residual mix, ``sssd_norm`` -> SSSD, ``cham_norm`` ->
 CHAM, ``mcmoe_norm`` -> M-CMoE), with ``SSSDAttention`` and ``ContinuousHolographicMemory``
-running on the HIP kernels and the M-CMoE as torch ops.  ``VeraceV1Model`` restates the
+running on the HIP kernels, the M-CMoE's products on the library and the steps between all
+of them fused in inference (:mod:`verace_amd.layer_ops`).  ``VeraceV1Model`` restates the
 text path of ``backbone.py:104-210`` (embedding tied to ``lm_head``, the layers, ACDE or the
 static loop, final norm); the vision encoder and the energy critic are not built (images are
 out of scope; ``vision_encoder.*`` / ``energy_critic.*`` keys are ignored when loading a
